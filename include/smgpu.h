@@ -308,7 +308,7 @@ int sm_mesher_destroy(sm_mesher *m);
  * (3D re-tetrahedralises at every triangulation step). */
 int sm_mesher_set_points(sm_mesher *m, const double *p, int64_t n);
 /* Runs `iters` force iterations (each: triangulation repair in 2D or an
- * exact host re-tetrahedralisation in 3D, centroid filter, unique edges,
+ * exact re-tetrahedralisation in 3D, centroid filter, unique edges,
  * bar forces, update, projection).  `maxdp_out`
  * (host, may be NULL) receives the last iteration's max movement. */
 int sm_mesher_run(sm_mesher *m, int iters, double *maxdp_out);
@@ -330,22 +330,22 @@ int sm_mesher_get_edges(sm_mesher *m, int32_t *edges, int64_t cap);
  * the slot count or an error code.  For checking the device repair. */
 int64_t sm_mesher_get_triangulation(sm_mesher *m, int32_t *tri, int32_t *adj, int64_t cap);
 /* Statistics since creation: [0] iterations, [1] flip rounds, [2] flips,
- * [3] host rebuilds (every 3D triangulation is one), [4] exact predicate
+ * [3] rebuilds (on the host in 2D; every 3D triangulation is one), [4] exact predicate
  * evaluations, [5] speculative (graph) iterations redone because their flips
  * had not converged, [6] kinetic repairs (points moved in sub-steps from the
  * last valid triangulation), [7] predicates the device's exact stage could
  * not settle (each forces a host rebuild), [8] vertices taken out and put
- * back on the host to untangle what flips could not, [9] 3D builds on
- * several threads, [10] points the threads left to the final single-thread
+ * back on the host to untangle what flips could not, [9] 3D builds on the
+ * device or on several host threads, [10] points the threads left to the final single-thread
  * pass (their cells were locked by another thread twice), [11] finite
  * tetrahedra of the last 3D build (0 in 2D), [12]
- * microseconds spent in the host 3D tetrahedralisation (wall clock, copies
- * and overlapped filters included). */
+ * microseconds spent in the 3D tetrahedralisation (wall clock; on the host
+ * with copies and overlapped filters). */
 int sm_mesher_stats(sm_mesher *m, int64_t *stats, int nstats);
-/* 3D handles: build each iteration's tetrahedralisation on nthreads host
- * threads inserting the points of nslabs slabs along `axis` into one shared
- * tetrahedralisation (sm_host_delaunay3d_slabs: the serial build's cells);
- * its cells are copied to the device and filtered there, piece by piece, on
+/* 3D handles: what the device build leaves to the host (small or degenerate
+ * point sets) is tetrahedralised on nthreads host threads inserting the points of nslabs slabs along `axis` into one shared
+ * tetrahedralisation (sm_host_delaunay3d_slabs: the serial build's cells, as
+ * the device's are); its cells are copied to the device and filtered there, piece by piece, on
  * the handle's stream while the host still hands out the next pieces.
  * Replaces the per-rank slabs of mesh_generator.py:808-852, :867-877 and
  * decomp/blocker.py:4-111 (axis as the reference's `axis` option). */

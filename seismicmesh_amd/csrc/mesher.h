@@ -8,6 +8,7 @@
 #include "common.h"
 #include "delaunay3d.h"
 #include "sizing_eval.h"
+#include "stars3d.h"
 
 constexpr int kNumStats = 13;
 
@@ -153,11 +154,13 @@ struct sm_mesher {
   int64_t dnn_cap = 0;
   uint64_t *d_sg = nullptr;
 
-  // 3D: the host tetrahedralisation, built by sl_threads threads inserting
-  // the points of sl_n slabs along sl_axis into one shared
-  // tetrahedralisation (delaunay3d.cpp); its cells are copied to the device
-  // and filtered there piece by piece while the host hands out the next.
+  // 3D: the tetrahedralisation is built on the device (stars3d.hip).  What
+  // that leaves to the host is built by sl_threads threads inserting the
+  // points of sl_n slabs along sl_axis into one shared tetrahedralisation
+  // (delaunay3d.cpp); its cells are copied to the device piece by piece
+  // while the host hands out the next, and filtered there.
   int sl_axis = 1, sl_n = 1, sl_threads = 1;
+  smk::StarScratch stars;
   smdt::DT3 dt3;
   double *h_pts = nullptr;  // pinned staging of the points (N, 3)
   int32_t *h_tet = nullptr;  // pinned staging of the tetrahedra (capT, 4)

@@ -174,8 +174,27 @@ int host_sizing_pass(sm_mesher *m) {
   return SM_OK;
 }
 
-// 3D: the tetrahedralisation is rebuilt on the host from the current points
-// every iteration (as the reference does with CGAL), on sl_threads threads
+// 3D: the tetrahedralisation is rebuilt from the current points every
+// iteration (as the reference does with CGAL), on the device (stars3d.hip).
+// *done is false when the device leaves it to host_rebuild3d.
+int device_rebuild3d(sm_mesher *m, bool *done) {
+  const auto t0 = std::chrono::steady_clock::now();
+  int64_t count = 0;
+  int rc = device_delaunay3d(&m->stars, m->d_p, m->N, m->prm.h0, m->d_tri, m->capT, &count, done,
+                             m->stream);
+  if (rc || !*done) return rc;
+  m->T = count;
+  m->stats[3] += 1;
+  m->stats[9] += 1;
+  m->stats[11] = count;
+  m->have_tri = true;
+  m->stats[12] += (int64_t)std::chrono::duration_cast<std::chrono::microseconds>(
+                      std::chrono::steady_clock::now() - t0)
+                      .count();
+  return SM_OK;
+}
+
+// 3D on the host, where the device build declines: on sl_threads threads
 // inserting the points of sl_n slabs into one shared tetrahedralisation.
 // Its cells are sorted straight into pinned staging and handed out in
 // pieces, each copied to the device asynchronously as it comes; the
@@ -258,9 +277,10 @@ int host_rebuild3d(sm_mesher *m, bool *filtered) {
 int triangulate(sm_mesher *m) {
   m->nsl = -1;  // a sliver selection refers to the previous cells
   if (m->dim == 3) {
-    bool filtered = false;
-    int rc = host_rebuild3d(m, &filtered);
+    bool built = false, filtered = false;
+    int rc = device_rebuild3d(m, &built);
     if (rc) return rc;
+    if (!built && (rc = host_rebuild3d(m, &filtered))) return rc;
     if (!filtered) {
       int b = prof_begin(m);
       rc = centroid_keep(m);
@@ -521,6 +541,7 @@ extern "C" int sm_mesher_destroy(sm_mesher *m) {
   dfree(m->d_bands);
   if (m->h_pts) (void)hipHostFree(m->h_pts);
   if (m->h_tet) (void)hipHostFree(m->h_tet);
+  stars_free(&m->stars);
   for (hipEvent_t e : m->ev_pool) (void)hipEventDestroy(e);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;

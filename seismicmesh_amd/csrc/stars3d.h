@@ -1,0 +1,41 @@
+// Device 3D Delaunay tetrahedralisation, one vertex star per wave
+// (stars3d.hip).
+#pragma once
+
+#include <cstdint>
+#include <vector>
+
+#include "common.h"
+
+namespace smk {
+
+// Scratch of the device build (one per handle, sized for its points).
+struct StarScratch {
+  int64_t cap_n = 0;
+  void *mem = nullptr;
+  size_t bytes = 0;
+  int32_t *h_status = nullptr;  // pinned
+  int skip = 0;                 // builds left to the host after a failed one
+  int64_t builds = 0, hubs = 0;
+};
+
+void stars_free(StarScratch *s);
+
+// Fewest points the device build takes on.  Its launches and the longest
+// chain of dependent insertions take 0.5-0.7 ms whatever the size; the
+// host's serial build takes 2 us a point (100 points: 0.2 ms against 0.65;
+// 1000: 2.1 against 0.9).
+constexpr int64_t kStarMinPoints = 512;
+
+// The finite Delaunay tetrahedra of the n points p (device, (n, 3) FP64) to
+// `tet` (device, room for cap cells): the same cells in the same order as
+// sm_host_delaunay3d.  `spacing` is a typical distance between neighbouring
+// points (any positive value is correct; it sizes the search grid).
+// Synchronises the stream.  *done is false when the device leaves the build
+// to the host (too few points, points in one plane, predicates its exact
+// stage cannot settle, too many uncertain ones or very large stars); nothing is
+// written then that the host build does not replace.
+int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacing, int32_t *tet,
+                      int64_t cap, int64_t *count, bool *done, hipStream_t s);
+
+}  // namespace smk

@@ -1,0 +1,125 @@
+"""The device tetrahedralisation (csrc/stars3d.hip) against the host's:
+the same cells in the same order, as integers, for every kind of point set
+that takes another way through it (the tolerance is equality)."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    from seismicmesh_amd import _lib
+    _lib.require_gpu()
+
+
+def _host(p):
+    from seismicmesh_amd import _lib
+    n = len(p)
+    t = np.empty((40 * n + 64, 4), dtype=np.int32)
+    ins = np.empty(n, dtype=np.uint8)
+    m = _lib.lib.sm_host_delaunay3d(p.ctypes.data, n, t.ctypes.data, len(t), ins.ctypes.data)
+    assert m >= 0
+    return t[:m]
+
+
+def _device(p, h):
+    """Every cell of the handle's tetrahedralisation (a domain that holds
+    them all), and whether the device built it."""
+    from seismicmesh_amd import generation, geometry as geo
+    lo, hi = p.min(0), p.max(0)
+    dom = geo.Ball([float(v) for v in (lo + hi) / 2], 1e7 * float((hi - lo).max()))
+    m = generation.Mesher([dom], generation._Sizing("const", value=h), h, 0.2, 0.1 * h, 1e-8 * h,
+                          0, precision=32, dim=3)
+    m.set_points(p)
+    m.triangulate()
+    s = m.stats()
+    t = m.cells()
+    m.close()
+    assert s["host_rebuilds"] == 1
+    return t, s["parallel_builds"] == 1
+
+
+def _box(rng, n, noise):
+    # a jittered lattice whose outer layers lie in the six sides of a box,
+    # exactly or up to rounding noise
+    g = np.linspace(0.0, 1.0, n)
+    p = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+    side = (p == 0.0) | (p == 1.0)
+    p = p + np.where(side, noise * rng.uniform(-1, 1, p.shape),
+                     rng.uniform(-0.2, 0.2, p.shape) / n)
+    return p
+
+
+def _points(kind):
+    rng = np.random.default_rng(11)
+    if kind.startswith("random"):
+        n = int(kind[6:])
+        return rng.uniform(-1, 1, (n, 3)), 2.0 / n ** (1 / 3)
+    if kind == "spacing_too_large":
+        return rng.uniform(-1, 1, (2000, 3)), 1e3
+    if kind == "spacing_too_small":
+        return rng.uniform(-1, 1, (2000, 3)), 1e-7
+    if kind == "clustered":
+        return np.vstack([rng.normal(0, 0.02, (1500, 3)), rng.uniform(-1, 1, (1500, 3))]), 0.02
+    if kind == "box_exact":
+        return _box(rng, 13, 0.0), 1 / 12
+    if kind == "box_noise":
+        return _box(rng, 13, 1e-15), 1 / 12
+    if kind == "duplicates":
+        p = rng.uniform(-1, 1, (1500, 3))
+        return np.vstack([p, p[::7], p[::11]]), 0.15
+    if kind == "hub":
+        # one point amid many at nearly one distance: a star of hundreds
+        # of cells, left to its neighbours
+        d = rng.normal(size=(700, 3))
+        d *= (1.0 + 1e-3 * rng.uniform(-1, 1, (700, 1))) / np.linalg.norm(d, axis=1)[:, None]
+        return np.vstack([rng.normal(0, 1e-3, (3, 3)), d, 3.0 * rng.uniform(-1, 1, (900, 3))]), 0.3
+    if kind == "long":
+        return rng.uniform(0, 1, (3000, 3)) * np.array([400.0, 1.0, 1.0]), 0.5
+    if kind == "far_from_origin":
+        return rng.uniform(0, 1, (2000, 3)) + 1e6, 0.08
+    if kind == "tiny":
+        return rng.uniform(0, 1, (2000, 3)) * 1e-9, 0.08e-9
+    if kind == "lattice":
+        g = np.arange(12) * 0.1
+        return np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3), 0.1
+    assert kind == "plane"
+    return np.column_stack([rng.uniform(0, 1, (200, 2)), np.zeros(200)]), 0.1
+
+
+@pytest.mark.parametrize("kind", [
+    "random511", "random512", "random513", "random2000", "random30000", "spacing_too_large",
+    "spacing_too_small", "clustered", "box_exact", "box_noise", "duplicates", "hub", "long",
+    "far_from_origin", "tiny", "lattice", "plane"])
+def test_cells_equal_the_host_build(kind):
+    p, h = _points(kind)
+    p = np.ascontiguousarray(p)
+    ref = _host(p)
+    got, on_device = _device(p, h)
+    assert np.array_equal(got, ref)
+    if kind.startswith("random") or kind in ("box_exact", "box_noise", "hub", "long",
+                                             "duplicates"):
+        assert on_device == (len(p) >= 512)
+    if kind == "plane":
+        assert len(ref) == 0 and not on_device
+
+
+def test_a_failed_build_is_followed_by_the_host_then_the_device_again():
+    """One handle over point sets that the device build takes, leaves to the
+    host, and takes again: each triangulation is that of its own points."""
+    from seismicmesh_amd import generation, geometry as geo
+    rng = np.random.default_rng(5)
+    g = np.arange(11) * 0.1
+    lat = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+    m = generation.Mesher([geo.Ball([0.0, 0.0, 0.0], 1e7)],
+                          generation._Sizing("const", value=0.1), 0.1, 0.2, 0.01, 1e-9, 0,
+                          precision=32, dim=3)
+    for p in [lat + rng.uniform(-0.02, 0.02, lat.shape), lat] + \
+             [lat + rng.uniform(-0.02, 0.02, lat.shape) for _ in range(5)]:
+        m.set_points(p)
+        m.triangulate()
+        assert np.array_equal(m.cells(), _host(np.ascontiguousarray(p)))
+    assert m.stats()["parallel_builds"] >= 2
+    m.close()
