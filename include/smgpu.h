@@ -150,8 +150,23 @@ int sm_mlp_eval(const sm_mlp *net, const double *x, int64_t n, float *d, void *s
 int sm_mlp_eval_centroids(const sm_mlp *net, const int32_t *cells, int64_t ncells,
                           const double *p, float *d, void *stream);
 
-/* Training kernels (FP32).  The forward and backward passes of the
- * network are sequences of these calls on caller-owned buffers.
+/* One training pass (FP32): the loss of sm_mlp_sdf_loss over n samples x
+ * ((n, in_dim) FP64, device) with targets t (FP32, device), and its gradient
+ * with respect to the network's flat FP32 parameters (device): w_in
+ * [width][in_dim], b_in [width], w_hid [hidden][width][width] (rows = output
+ * features), b_hid [hidden][width], w_out [width], b_out [1]; width is 256,
+ * hidden at most 16.  shift and scale are host arrays of in_dim values.
+ * eik_h > 0: the central-difference eikonal term with step eik_h and weight
+ * lam.  grad: as many values as params; part: ceil(n / 256) loss partials.
+ * params and ws are 16-byte aligned; ws holds at least
+ * sm_mlp_loss_grad_workspace bytes (0 for bad sizes). */
+size_t sm_mlp_loss_grad_workspace(int64_t n, int in_dim, int hidden, float eik_h);
+int sm_mlp_loss_grad(int64_t n, int in_dim, int hidden, const double *x, const float *t,
+                     const double *shift, const double *scale, float eik_h, float lam,
+                     float trunc, const float *params, float *grad, float *part, void *ws,
+                     size_t ws_bytes, void *stream);
+
+/* The same pass in single steps, on caller-owned buffers.
  *
  * C[m, n] = alpha * sum_k A(m, k) B(k, n) + beta * C[m, n] with
  * A(m, k) = A[m * sam + k * sak], B(k, n) = B[k * sbk + n * sbn] and C

@@ -9,16 +9,17 @@
 // 32x32x16 product); a hidden layer is 8 column blocks x 16 k-steps, whose
 // weight fragments the workgroup's 8 waves share through LDS.
 //
-// Training uses FP32 kernels: a tiled GEMM with strided operands and an
-// optional deterministic split over k (forward X W^T, backward dZ W,
-// weight gradients dZ^T X), bias + SiLU, its derivative, the loss with a
-// central-difference eikonal term, and Adam.
+// Training uses FP32 kernels: the fused pass of mlp_train.hip, and here its
+// loss with a central-difference eikonal term, Adam, and the single steps
+// (a tiled GEMM with strided operands and an optional deterministic split
+// over k, bias + SiLU, its derivative).
 //
 // The reference has no counterpart: it evaluates the CSG functions of
 // signed_distance_functions.py:283-623 directly.
 #include <cmath>
 
 #include "common.h"
+#include "mlp_gemm.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
@@ -533,6 +534,41 @@ extern "C" int sm_gemm_f32(int M, int N, int K, float alpha, const float *A, int
   const int ns = nsplit == 1 ? 1 : (K + kchunk - 1) / kchunk;
   const int nz = ns > 0 ? ns : 1;
   hipStream_t s = stream_of(stream);
+  // One index of each operand contiguous, 16-byte aligned runs, and more
+  // than a sliver of a tile: the matrix cores (57344 x 256 x 256: 0.09 ms
+  // against 1.0 here).  Products with one or a few rows or columns stay on
+  // the vector kernel, which any strides suit.
+  {
+    GemmArgs a;
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    a.A = A;
+    a.B = B;
+    const bool ak = sak == 1, bk = sbk == 1;
+    a.lda = ak ? sam : sak;
+    a.ldb = bk ? sbn : sbk;
+    const bool unit = (ak || sam == 1) && (bk || sbn == 1);
+    if (unit && M >= 32 && N >= 32 && gemm32_takes(ak, bk, a)) {
+      const bool small = (int64_t)((M + 127) / 128) * ((N + 127) / 128) * nsplit < 256;
+      if (nsplit == 1) {
+        a.C = C;
+        a.ldc = ldc;
+        a.alpha = alpha;
+        a.beta = beta;
+        return gemm32(kEpiStore, ak, bk, a, small, s);
+      }
+      a.C = work;
+      a.ldc = N;
+      a.nsplit = nsplit;
+      int rc = gemm32(kEpiPart, ak, bk, a, small, s);
+      if (rc) return rc;
+      hipLaunchKernelGGL(k_split_reduce, dim3(blocks_for((int64_t)M * N, 256)), dim3(256), 0, s,
+                         M, N, gemm32_splits(a), work, alpha, beta, C, ldc);
+      SM_LAUNCH_CHECK();
+      return SM_OK;
+    }
+  }
   dim3 g((N + kGT - 1) / kGT, (M + kGT - 1) / kGT, nz);
   hipLaunchKernelGGL(k_gemm_f32, g, dim3(256), 0, s, M, N, K, kchunk, alpha, A, sam, sak, B, sbk,
                      sbn, beta, C, ldc, nsplit == 1 ? nullptr : work);

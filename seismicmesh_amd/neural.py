@@ -4,9 +4,8 @@ SeismicMesh/geometry/signed_distance_functions.py:283-623).
 
 NeuralSDF is a multilayer perceptron dim -> 256 -> ... -> 256 -> 1 with
 SiLU activations.  It is trained on the GPU by libsmgpu's own FP32 kernels
-(sm_gemm_f32 for the forward and backward products, sm_mlp_bias_silu,
-sm_mlp_silu_backward, sm_mlp_sdf_loss, sm_mlp_adam) on samples of the
-domain's exact SDF -- half uniform in the bounding box, half within `near`
+(sm_mlp_loss_grad: the forward and backward pass; sm_mlp_adam) on samples of
+the domain's exact SDF -- half uniform in the bounding box, half within `near`
 of the surface -- with the squared error plus a central-difference eikonal
 term.  Inference (sm_mlp_eval) is the fused BF16 matrix-core kernel.
 
@@ -113,10 +112,6 @@ class NeuralSDF:
         self.trunc = None
         self._bufs = {}
         self._dirty = True
-        self._shift_d = torch.tensor(np.r_[self.shift, 0.0][:3], dtype=torch.float64,
-                                     device=self.dev)
-        self._scale_d = torch.tensor(np.r_[self.scale, 0.0][:3], dtype=torch.float64,
-                                     device=self.dev)
 
     # ------------------------------------------------------------ helpers
     def _stream(self):
@@ -192,31 +187,14 @@ class NeuralSDF:
         return out.cpu().numpy()
 
     # ----------------------------------------------------------- training
-    def _buffers(self, n, eik):
-        rows = n * (2 * self.dim + 1 if eik else 1)
-        key = (n, bool(eik))
-        if key in self._bufs:
-            return self._bufs[key]
-        torch, W, L = self.torch, self.width, self.hidden
-        f32 = dict(dtype=torch.float32, device=self.dev)
-        nsplit = int(max(1, min(64, rows // 2048)))
-        b = dict(rows=rows, nsplit=nsplit,
-                 X=torch.empty(rows * self.dim, **f32),
-                 Z=[torch.empty(rows * W, **f32) for _ in range(L + 1)],
-                 A=[torch.empty(rows * W, **f32) for _ in range(L + 1)],
-                 dA=torch.empty(rows * W, **f32), dZ=torch.empty(rows * W, **f32),
-                 y=torch.empty(rows, **f32), gy=torch.empty(rows, **f32),
-                 ones=torch.from_numpy(np.ones(rows, dtype=np.float32)).to(self.dev),
-                 part=torch.empty((n + 255) // 256, **f32),
-                 work=torch.empty(nsplit * W * W + 16, **f32))
-        self._bufs = {key: b}  # keep one set
-        return b
-
-    def _gemm(self, M, N, K, A, sam, sak, B, sbk, sbn, C, ldc, nsplit=1, work=None,
-              alpha=1.0, beta=0.0):
-        _lib.check(_lib.lib.sm_gemm_f32(M, N, K, alpha, A, sam, sak, B, sbk, sbn, beta, C, ldc,
-                                        nsplit, work if work is not None else None,
-                                        self._stream()), "sm_gemm_f32")
+    def _buffers(self, n, eik_h):
+        key = (n, eik_h > 0)
+        if key not in self._bufs:
+            size = _lib.lib.sm_mlp_loss_grad_workspace(n, self.dim, self.hidden, eik_h)
+            ws = self.torch.empty(max(size, 16), dtype=self.torch.uint8, device=self.dev)
+            part = self.torch.empty((n + 255) // 256, dtype=self.torch.float32, device=self.dev)
+            self._bufs = {key: (ws, part)}  # keep one set
+        return self._bufs[key]
 
     def loss_and_grad(self, xt, tt, eik=0.1, eik_h=5e-3, trunc=0.0):
         """Forward and backward pass over the samples xt ((n, dim) float64
@@ -225,59 +203,14 @@ class NeuralSDF:
         eikonal term is dropped).  Fills self.grad; returns the loss
         partials (device)."""
         n = xt.shape[0]
-        W, L, dim = self.width, self.hidden, self.dim
-        b = self._buffers(n, eik > 0)
-        rows, nsplit, work = b["rows"], b["nsplit"], _ptr(b["work"])
-        st = self._stream()
-        _lib.check(_lib.lib.sm_mlp_make_inputs(n, dim, _ptr(xt), _ptr(self._shift_d),
-                                               _ptr(self._scale_d),
-                                               float(eik_h) if eik > 0 else 0.0,
-                                               _ptr(b["X"]), st), "sm_mlp_make_inputs")
-        Z, A = b["Z"], b["A"]
-        # forward: Z0 = X W_in^T, A_l = silu(Z_l + b_l), y = A_L w_out + b_out
-        self._gemm(rows, W, dim, _ptr(b["X"]), dim, 1, self._p("w_in"), 1, dim, _ptr(Z[0]), W)
-        _lib.check(_lib.lib.sm_mlp_bias_silu(rows, W, _ptr(Z[0]), self._p("b_in"), _ptr(A[0]),
-                                             st), "sm_mlp_bias_silu")
-        woff = self.layout["w_hid"][0]
-        boff = self.layout["b_hid"][0]
-        for l in range(1, L + 1):
-            Wl = _ptr(self.params, woff + (l - 1) * W * W)
-            self._gemm(rows, W, W, _ptr(A[l - 1]), W, 1, Wl, 1, W, _ptr(Z[l]), W)
-            _lib.check(_lib.lib.sm_mlp_bias_silu(rows, W, _ptr(Z[l]),
-                                                 _ptr(self.params, boff + (l - 1) * W),
-                                                 _ptr(A[l]), st), "sm_mlp_bias_silu")
-        self._gemm(rows, 1, W, _ptr(A[L]), W, 1, self._p("w_out"), 1, 0, _ptr(b["y"]), 1)
-        _lib.check(_lib.lib.sm_mlp_bias_silu(rows, 1, _ptr(b["y"]), self._p("b_out"), None, st),
-                   "sm_mlp_bias_silu")
-        _lib.check(_lib.lib.sm_mlp_sdf_loss(n, dim, _ptr(b["y"]), _ptr(tt), float(eik_h),
-                                            float(eik), float(trunc), _ptr(b["gy"]),
-                                            _ptr(b["part"]), st),
-                   "sm_mlp_sdf_loss")
-        g = self.grad
-        gy = _ptr(b["gy"])
-        # output layer: dw_out = gy^T A_L, db_out = sum gy, dA_L = gy w_out^T
-        self._gemm(1, W, rows, gy, 0, 1, _ptr(A[L]), W, 1, self._p("w_out", g), W, nsplit, work)
-        self._gemm(1, 1, rows, gy, 0, 1, _ptr(b["ones"]), 1, 0, self._p("b_out", g), 1, nsplit,
-                   work)
-        self._gemm(rows, W, 1, gy, 1, 0, self._p("w_out"), 0, 1, _ptr(b["dA"]), W)
-        for l in range(L, -1, -1):
-            _lib.check(_lib.lib.sm_mlp_silu_backward(rows * W, _ptr(Z[l]), _ptr(b["dA"]),
-                                                     _ptr(b["dZ"]), st), "sm_mlp_silu_backward")
-            dZ = _ptr(b["dZ"])
-            if l == 0:
-                self._gemm(W, dim, rows, dZ, 1, W, _ptr(b["X"]), dim, 1, self._p("w_in", g), dim,
-                           nsplit, work)
-                self._gemm(1, W, rows, _ptr(b["ones"]), 0, 1, dZ, W, 1, self._p("b_in", g), W,
-                           nsplit, work)
-                break
-            # dW_l = dZ_l^T A_{l-1}, db_l = sum_rows dZ_l, dA_{l-1} = dZ_l W_l
-            self._gemm(W, W, rows, dZ, 1, W, _ptr(A[l - 1]), W, 1,
-                       _ptr(g, woff + (l - 1) * W * W), W, nsplit, work)
-            self._gemm(1, W, rows, _ptr(b["ones"]), 0, 1, dZ, W, 1, _ptr(g, boff + (l - 1) * W),
-                       W, nsplit, work)
-            self._gemm(rows, W, W, dZ, W, 1, _ptr(self.params, woff + (l - 1) * W * W), W, 1,
-                       _ptr(b["dA"]), W)
-        return b["part"]
+        step = float(eik_h) if eik > 0 else 0.0
+        ws, part = self._buffers(n, step)
+        _lib.check(_lib.lib.sm_mlp_loss_grad(
+            n, self.dim, self.hidden, _ptr(xt), _ptr(tt), self.shift.ctypes.data,
+            self.scale.ctypes.data, step, float(eik), float(trunc), _ptr(self.params),
+            _ptr(self.grad), _ptr(part), _ptr(ws), ws.numel(), self._stream()),
+            "sm_mlp_loss_grad")
+        return part
 
     def adam_step(self, lr, b1=0.9, b2=0.999, eps=1e-8):
         self.step += 1

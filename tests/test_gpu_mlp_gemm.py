@@ -1,0 +1,78 @@
+"""The matrix-core product behind sm_gemm_f32 and the fused training pass."""
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def gpu():
+    from seismicmesh_amd import _lib
+    _lib.require_gpu()
+
+
+def _p(t):
+    return ctypes.c_void_p(t.data_ptr())
+
+
+# edges of the 64 and 128 tiles and of the 16-deep slices, every layout, with
+# and without a split; the last ones fall back to the vector kernel (rows too
+# few, an unaligned stride, a stride below the run: overlapping rows)
+@pytest.mark.parametrize("M,N,K,ta,tb,nsplit,off", [
+    (64, 64, 16, False, False, 1, 0), (68, 60, 20, False, False, 1, 0),
+    (128, 128, 16, True, False, 1, 0), (132, 124, 36, True, True, 1, 0),
+    (256, 256, 4, False, True, 1, 0), (33, 256, 256, False, True, 1, 0),
+    (256, 256, 5001, True, False, 7, 0), (256, 256, 17, True, False, 9, 0),
+    (16500, 256, 256, False, True, 1, 0), (16384, 260, 64, False, False, 3, 0),
+    (31, 256, 256, False, True, 1, 0), (256, 256, 30, False, True, 1, 0),
+    (64, 64, 64, False, True, 1, 1)])
+def test_gemm_matches_float64(M, N, K, ta, tb, nsplit, off):
+    import torch
+    from seismicmesh_amd import _lib
+    rng = np.random.default_rng(M + N + K)
+    A = rng.standard_normal((K, M) if ta else (M, K)).astype(np.float32)
+    B = rng.standard_normal((N, K) if tb else (K, N)).astype(np.float32)
+    C0 = rng.standard_normal((M, N)).astype(np.float32)
+    dev = "cuda:0"
+    Ad = torch.empty(A.size + off, dtype=torch.float32, device=dev)
+    Ad[off:] = torch.from_numpy(A).to(dev).reshape(-1)
+    Bd, Cd = torch.from_numpy(B).to(dev), torch.from_numpy(C0).to(dev)
+    work = torch.empty(nsplit * M * N, dtype=torch.float32, device=dev)
+    sam, sak = (1, M) if ta else (K, 1)
+    sbk, sbn = (1, K) if tb else (N, 1)
+    _lib.check(_lib.lib.sm_gemm_f32(M, N, K, 0.5, _p(Ad[off:]), sam, sak, _p(Bd), sbk, sbn, 2.0,
+                                    _p(Cd), N, nsplit, _p(work), None), "sm_gemm_f32")
+    torch.cuda.synchronize()
+    Am, Bm = (A.T if ta else A).astype(np.float64), (B.T if tb else B).astype(np.float64)
+    got = Cd.cpu().numpy()
+    # each output: K roundings of its own partial sums at most, and four more
+    bound = 2.0 ** -24 * (K + 4) * (0.5 * np.abs(Am) @ np.abs(Bm) + 2.0 * np.abs(C0))
+    assert (np.abs(got - (0.5 * (Am @ Bm) + 2.0 * C0)) <= bound).all()
+
+
+# row counts around the tile sizes and the switch between them (16384 rows),
+# with and without the eikonal copies, no hidden layer at all
+@pytest.mark.parametrize("n,dim,hidden,lam", [
+    (1, 3, 1, 0.0), (63, 2, 2, 0.0), (65, 3, 3, 0.1), (300, 2, 0, 0.1), (2341, 3, 1, 0.1),
+    (16383, 2, 1, 0.0), (16385, 3, 2, 0.0)])
+def test_training_pass_matches_float64(n, dim, hidden, lam):
+    import torch
+    from oracle import mlp as omlp
+    from seismicmesh_amd.neural import NeuralSDF
+    net = NeuralSDF(dim, [-1.0, 1.0] * dim, hidden=hidden, seed=3)
+    rng = np.random.default_rng(n)
+    x = rng.uniform(-1, 1, (n, dim))
+    t = (np.linalg.norm(x, axis=1) - 0.5).astype(np.float32)
+    part = net.loss_and_grad(torch.from_numpy(x).cuda(), torch.from_numpy(t).cuda(), eik=lam)
+    g = net.grad.cpu().numpy().astype(np.float64)
+    L, ref = omlp.loss_and_grad(net.numpy_params().astype(np.float64), dim, 256, hidden, x,
+                                t.astype(np.float64), net.shift, net.scale, lam=lam, eik_h=5e-3)
+    assert abs(float(part.cpu().numpy().astype(np.float64).sum()) - L) <= 1e-4 * abs(L)
+    for name, (o, k) in net.layout.items():
+        if k == 0:
+            continue
+        r = ref[o:o + k]
+        # as test_training_gradient_matches_oracle
+        assert np.abs(g[o:o + k] - r).max() <= 2e-3 * np.abs(r).max() + 1e-7, name
