@@ -362,7 +362,7 @@ __device__ __noinline__ int insphere_exact_call(P3 a, P3 b, P3 c, P3 d, P3 e) {
 // ------------------------------------------------------------- the stars
 constexpr int kInfV = 0xffff;  // the vertex at infinity in a triangle
 constexpr int kDead = -1;      // an unused triangle slot (in .a)
-constexpr int kTab = 112;      // points inserted into one link, replaced ones included
+constexpr int kTab = 64;       // points held for one link
 constexpr int kStack = 64 * kMaxLevels;
 
 __device__ inline void wave_sync() {
@@ -391,6 +391,7 @@ struct StarLds {
   double cx[64], cy[64], cz[64];        // candidates of a chunk
   int32_t ci[64];
   int32_t run0[64], runp[64];  // runs of grid points, inclusive prefix of lengths
+  int32_t used[kTab];
   uint32_t rim[66];            // directed edges of a hole's rim
 };
 struct FarLds {
@@ -558,11 +559,25 @@ struct Star {
     return kOk;
   }
 
+  // a table entry no triangle refers to (64 triangles have at most 34
+  // vertices)
+  __device__ int recycle() {
+    const int lane = lane_of();
+    sh.used[lane] = 0;
+    wave_sync();
+    if (t.a != kDead) {
+      sh.used[t.a] = 1;
+      sh.used[t.b] = 1;
+      if (t.c != kInfV) sh.used[t.c] = 1;
+    }
+    wave_sync();
+    return __builtin_ctzll(__ballot(sh.used[lane] == 0));
+  }
+
   // the triangles in conf replaced by the cone from (x, y, z)
   __device__ int insert(double x, double y, double z, int32_t idx) {
-    if (ntab >= kTab) return kOverflow;
     const int lane = lane_of();
-    const int q = ntab++;
+    const int q = ntab < kTab ? ntab++ : recycle();
     if (lane == 0) {
       sh.tx[q] = x;
       sh.ty[q] = y;
