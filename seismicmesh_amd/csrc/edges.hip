@@ -7,16 +7,18 @@
 // Method: the sort key of an edge is (min, max) with min a vertex id, so the
 // lexicographic sort is a counting sort on min (one bucket per vertex: a
 // histogram, an exclusive scan and a scatter) followed by a sort of each
-// bucket's max ids.  Buckets hold a vertex's higher neighbours (a handful in
-// a 2D mesh: sorted in one thread's registers; a few dozen in 3D, where an
-// edge comes once per incident cell: one wave, one id per lane); long
-// buckets (arbitrary user input) are sorted by a whole workgroup in LDS
-// or, beyond that, in global memory.
-// Duplicates are dropped inside each sorted bucket; a second scan turns the
-// per-bucket unique counts into output offsets.  For a 2D triangulation with
-// neighbour links each shared edge is produced once in the first place (by
-// the lower-numbered of its two cells) and the second scan is skipped.  The
-// output is exactly the reference's sorted unique edge list.
+// bucket's max ids.  Cells near each other in the list share most of their
+// edges, so a block first drops the duplicates among its own cells in LDS
+// and only what is left is counted and scattered.  Buckets then hold a
+// vertex's higher neighbours and few duplicates: up to 16 ids are sorted in
+// one thread's registers, up to 64 by one wave, one id per lane; long
+// buckets (arbitrary user input) by a whole workgroup in LDS or, beyond
+// that, in global memory.  The remaining duplicates are dropped inside each
+// sorted bucket; a second scan turns the per-bucket unique counts into
+// output offsets.  For a 2D triangulation with neighbour links each shared
+// edge is produced once in the first place (by the lower-numbered of its two
+// cells) and neither the LDS pass nor the second scan is needed.  The output
+// is exactly the reference's sorted unique edge list.
 #include "common.h"
 #include "edges.h"
 
@@ -24,138 +26,182 @@ namespace smk {
 
 namespace {
 
-__device__ inline void pair_of(const int32_t *pairs, int64_t i, int32_t &a, int32_t &b) {
-  int32_t u = pairs[2 * i], v = pairs[2 * i + 1];
-  a = u < v ? u : v;
-  b = u < v ? v : u;
-}
-
-// local edge j of a cell in the reference's order (mesh_generator.py:683-687)
-__device__ inline void cell_edge(const int32_t *cells, int64_t c, int dim, int j, int32_t &a,
-                                 int32_t &b) {
-  const int32_t *t = cells + c * (dim + 1);
-  int u, v;
-  switch (j) {
-    case 0: u = t[0]; v = t[1]; break;
-    case 1: u = t[1]; v = t[2]; break;
-    case 2: u = t[2]; v = t[0]; break;
-    case 3: u = t[0]; v = t[3]; break;
-    case 4: u = t[1]; v = t[3]; break;
-    default: u = t[2]; v = t[3]; break;
-  }
-  a = u < v ? u : v;
-  b = u < v ? v : u;
-}
-
-struct PairSrc {
-  const int32_t *pairs;
+// Cells of 2D triangulations with neighbour links: adj[3 c + k] is the cell
+// across the edge opposite local vertex k, or < 0.  An edge shared by two
+// kept cells is produced once, by the lower-numbered one, so every bucket is
+// free of duplicates and its offsets are the output offsets.
+struct LinkSrc {
   const int32_t *cells;
   const uint8_t *keep;  // optional cell mask
-  // optional (2D cells only): adj[3 c + k] is the cell across the edge
-  // opposite local vertex k, or < 0.  An edge shared by two kept cells is
-  // then produced once, by the lower-numbered one, so every bucket is free
-  // of duplicates and its offsets are the output offsets.
   const int32_t *adj;
-  int dim;
-  int64_t n;            // pairs, or cells
-  __device__ inline int per() const { return pairs ? 1 : (dim == 2 ? 3 : 6); }
+  int64_t n;
   __device__ inline bool get(int64_t i, int j, int32_t &a, int32_t &b) const {
-    if (pairs) {
-      pair_of(pairs, i, a, b);
-      return true;
-    }
     if (keep && !keep[i]) return false;
-    if (adj) {
-      // local edge j joins vertices j and (j + 1) % 3: opposite vertex (j + 2) % 3
-      const int32_t o = adj[3 * i + (j + 2) % 3];
-      if (o >= 0 && o < i && (!keep || keep[o])) return false;
-    }
-    cell_edge(cells, i, dim, j, a, b);
+    // local edge j joins vertices j and (j + 1) % 3: opposite vertex (j + 2) % 3
+    const int32_t o = adj[3 * i + (j + 2) % 3];
+    if (o >= 0 && o < i && (!keep || keep[o])) return false;
+    const int32_t u = cells[3 * i + j], v = cells[3 * i + (j + 1) % 3];
+    a = u < v ? u : v;
+    b = u < v ? v : u;
     return true;
   }
 };
 
-// Tetrahedra: with the ids sorted, s0 < s1 < s2 < s3, the six edges are
-// three in bucket s0 (partners s1, s2, s3), two in bucket s1 (s2, s3) and
-// one in bucket s2 (s3): three contiguous runs instead of six pairs.  The
-// host tetrahedralisation hands out cells sorted by their lowest id, so
-// consecutive lanes share s0: the lanes of a run of equal s0 (consecutive,
-// all taking part) reserve their slots with one atomic by the run's first
-// lane.  Returns false for a lane without a cell.
-struct TetRun {
-  int32_t s[4];
-  bool ok, lead;
-  int len;    // lanes in the run (leader only)
-  int first;  // the run's first lane
+// Items without links: pairs (NV = 2), triangles (3) or tetrahedra (4).  A
+// block of kItemThreads threads takes kPer items a thread.
+struct ItemSrc {
+  const int32_t *ids;   // NV per item
+  const uint8_t *keep;  // optional mask
+  int64_t n;
+};
+constexpr int kItemThreads = 512;
+constexpr int kTable = 4096;  // LDS hash slots (vertices, pairs), 12 bits
+template <int NV>
+struct ItemShape {
+  static constexpr int pairs = NV == 2 ? 1 : (NV == 3 ? 3 : 6);
+  static constexpr int per = NV == 4 ? 1 : 2;
+  static constexpr int items = kItemThreads * per;
+  static constexpr int cap = items * pairs;  // pairs of one block
+  static_assert(cap <= kTable * 3 / 4 && items * NV <= kTable * 3 / 4, "tables stay 3/4 full");
 };
 
-__device__ inline TetRun tet_run(const PairSrc &src, int64_t i) {
-  TetRun r;
-  r.ok = i < src.n && (!src.keep || src.keep[i]);
-  if (r.ok) {
-    const int32_t *t = src.cells + 4 * i;
+__device__ inline uint32_t hash12(uint32_t x) { return (x * 2654435761u) >> 20; }
+
+// slot of v in an open-addressed LDS table (-1: empty), inserted if new.
+// Sixteen consecutive vertices start at consecutive slots, so that the
+// lanes that walk the table touch whole lines of the per-vertex arrays.
+__device__ inline int vertex_slot(int32_t *vk, int32_t v) {
+  uint32_t h = (hash12((uint32_t)v >> 4) & ~15u) | ((uint32_t)v & 15);
+  for (;;) {
+    int32_t o = vk[h];
+    if (o == v) return (int)h;
+    if (o == -1) o = atomicCAS(&vk[h], -1, v);
+    if (o == -1 || o == v) return (int)h;
+    h = (h + 1) & (kTable - 1);
+  }
+}
+
+// The distinct pairs among a block's items: vertices become their slot in an
+// LDS table (12 bits), a pair the 24-bit key of its two slots in a second
+// one.  The distinct pairs are appended to the block's segment of `list`
+// (cap pairs, see item_count for its length) and counted by first endpoint,
+// one global atomic per distinct endpoint of the block.
+// Bound by the atomics: 2.8 M lattice tetrahedra have 17 M pairs, 5 M after
+// this pass; counting and scattering runs of sorted ids straight from the
+// cells took 110 + 153 us, this pass and k_item_scatter 67 + 50 us.
+template <int NV>
+__global__ __launch_bounds__(kItemThreads) void k_item_count(ItemSrc src, int32_t *cnt,
+                                                            int2 *list) {
+  using S = ItemShape<NV>;
+  __shared__ int32_t vk[kTable], vc[kTable];
+  __shared__ uint32_t pk[kTable];
+  __shared__ int32_t npairs;
+  const int tid = threadIdx.x;
+  const int64_t blk = xcd_block();
+  for (int k = tid; k < kTable; k += kItemThreads) {
+    vk[k] = -1;
+    vc[k] = 0;
+    pk[k] = ~0u;
+  }
+  if (tid == 0) npairs = 0;
+  __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 4; ++k) r.s[k] = t[k];
-    // sorting network on four values
-#define SM_CSWAP(a, b)                      \
-  {                                         \
-    const int32_t x = r.s[a], y = r.s[b];   \
-    r.s[a] = x < y ? x : y;                 \
-    r.s[b] = x < y ? y : x;                 \
+  for (int it = 0; it < S::per; ++it) {
+    const int64_t i = blk * S::items + it * kItemThreads + tid;
+    if (i >= src.n || (src.keep && !src.keep[i])) continue;
+    int32_t v[NV];
+    int sl[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) v[k] = src.ids[NV * i + k];
+#pragma unroll
+    for (int k = 0; k < NV; ++k) sl[k] = vertex_slot(vk, v[k]);
+#pragma unroll
+    for (int x = 0; x < NV; ++x)
+#pragma unroll
+      for (int y = x + 1; y < NV; ++y) {
+        const uint32_t key =
+            v[x] < v[y] ? (uint32_t)(sl[x] << 12 | sl[y]) : (uint32_t)(sl[y] << 12 | sl[x]);
+        uint32_t h = hash12(key);
+        for (;;) {
+          uint32_t o = pk[h];
+          if (o == key) break;
+          if (o == ~0u) o = atomicCAS(&pk[h], ~0u, key);
+          if (o == ~0u || o == key) break;
+          h = (h + 1) & (kTable - 1);
+        }
+      }
   }
-    SM_CSWAP(0, 1) SM_CSWAP(2, 3) SM_CSWAP(0, 2) SM_CSWAP(1, 3) SM_CSWAP(1, 2)
-#undef SM_CSWAP
-  } else {
-    r.s[0] = r.s[1] = r.s[2] = r.s[3] = -1;
+  __syncthreads();
+  int2 *seg = list + blk * S::cap;
+  const int lane = tid % 64;
+  for (int k = tid; k < kTable; k += kItemThreads) {
+    const uint32_t key = pk[k];
+    const uint64_t m = __ballot(key != ~0u);
+    int32_t base = 0;
+    if (lane == 0 && m) base = atomicAdd(&npairs, (int32_t)__popcll(m));
+    base = __shfl(base, 0);
+    if (key != ~0u) {
+      atomicAdd(&vc[key >> 12], 1);
+      seg[base + (int32_t)__popcll(m & ((1ull << lane) - 1))] =
+          make_int2(vk[key >> 12], vk[key & (kTable - 1)]);
+    }
   }
-  const int lane = threadIdx.x % 64;
-  const int32_t prev = __shfl_up(r.s[0], 1);
-  const uint64_t okm = __ballot(r.ok);
-  const bool prev_ok = lane > 0 && ((okm >> (lane - 1)) & 1);
-  r.lead = r.ok && !(prev_ok && prev == r.s[0]);
-  const uint64_t brk = __ballot(!r.ok || r.lead);
-  const uint64_t after = lane == 63 ? 0 : brk >> (lane + 1);
-  r.len = after ? 1 + __builtin_ctzll(after) : 64 - lane;
-  const uint64_t starts = __ballot(r.lead) & (lane == 63 ? ~0ull : ((2ull << lane) - 1));
-  r.first = starts ? 63 - __builtin_clzll(starts) : lane;
-  return r;
+  __syncthreads();
+  for (int k = tid; k < kTable; k += kItemThreads)
+    if (vc[k]) atomicAdd(&cnt[vk[k]], vc[k]);
+  // the last segment is cut off at the last item
+  const int64_t left = src.n - blk * S::items;
+  const int32_t cap = (int32_t)(left < S::items ? left : S::items) * S::pairs;
+  if (tid == 0 && npairs < cap) seg[cap - 1] = make_int2(~npairs, 0);
 }
 
-__global__ void k_count_tets(PairSrc src, int32_t *cnt) {
-  const int64_t i = (int64_t)xcd_block() * blockDim.x + threadIdx.x;
-  const TetRun r = tet_run(src, i);
-  if (r.lead) atomicAdd(&cnt[r.s[0]], 3 * r.len);
-  if (r.ok) {
-    atomicAdd(&cnt[r.s[1]], 2);
-    atomicAdd(&cnt[r.s[2]], 1);
+// The listed pairs into their buckets: the block ranks its pairs by first
+// endpoint in LDS and reserves each bucket's slots with one global atomic.
+template <int NV>
+__global__ __launch_bounds__(kItemThreads) void k_item_scatter(int64_t n, const int2 *list,
+                                                              const int32_t *rowptr, int32_t *cur,
+                                                              int32_t *col) {
+  using S = ItemShape<NV>;
+  constexpr int R = S::cap / kItemThreads;
+  __shared__ int32_t vk[kTable], vc[kTable];
+  const int tid = threadIdx.x;
+  const int64_t blk = xcd_block();
+  if (blk * S::items >= n) return;
+  for (int k = tid; k < kTable; k += kItemThreads) {
+    vk[k] = -1;
+    vc[k] = 0;
   }
-}
-
-__global__ void k_scatter_tets(PairSrc src, const int32_t *rowptr, int32_t *cur,
-                               int32_t *col) {
-  const int64_t i = (int64_t)xcd_block() * blockDim.x + threadIdx.x;
-  const TetRun r = tet_run(src, i);
-  int32_t base = 0;
-  if (r.lead) base = rowptr[r.s[0]] + atomicAdd(&cur[r.s[0]], 3 * r.len);
-  base = __shfl(base, r.first);
-  if (!r.ok) return;
-  const int lane = threadIdx.x % 64;
-  const int32_t p0 = base + 3 * (lane - r.first);
-  col[p0] = r.s[1];
-  col[p0 + 1] = r.s[2];
-  col[p0 + 2] = r.s[3];
-  const int32_t p1 = rowptr[r.s[1]] + atomicAdd(&cur[r.s[1]], 2);
-  col[p1] = r.s[2];
-  col[p1 + 1] = r.s[3];
-  col[rowptr[r.s[2]] + atomicAdd(&cur[r.s[2]], 1)] = r.s[3];
+  const int2 *seg = list + blk * S::cap;
+  const int64_t left = n - blk * S::items;
+  const int32_t cap = (int32_t)(left < S::items ? left : S::items) * S::pairs;
+  // a segment that is not full ends with the complement of its length
+  const int32_t last = seg[cap - 1].x;
+  const int32_t m = last < 0 ? ~last : cap;
+  __syncthreads();
+  int32_t b[R], sl[R], rank[R];
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const int32_t e = k * kItemThreads + tid;
+    if (e >= m) continue;
+    const int2 pr = seg[e];
+    b[k] = pr.y;
+    sl[k] = vertex_slot(vk, pr.x);
+    rank[k] = atomicAdd(&vc[sl[k]], 1);
+  }
+  __syncthreads();
+  for (int k = tid; k < kTable; k += kItemThreads)
+    if (vc[k]) vc[k] = rowptr[vk[k]] + atomicAdd(&cur[vk[k]], vc[k]);
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < R; ++k)
+    if (k * kItemThreads + tid < m) col[vc[sl[k]] + rank[k]] = b[k];
 }
 
 // cnt2 (optional): the same edges counted by their second endpoint
-__global__ void k_count(PairSrc src, int32_t *cnt, int32_t *cnt2) {
+__global__ void k_count(LinkSrc src, int32_t *cnt, int32_t *cnt2) {
   int64_t i = (int64_t)xcd_block() * blockDim.x + threadIdx.x;
   if (i >= src.n) return;
-  const int per = src.per();
-  for (int j = 0; j < per; ++j) {
+  for (int j = 0; j < 3; ++j) {
     int32_t a, b;
     if (src.get(i, j, a, b)) {
       atomicAdd(&cnt[a], 1);
@@ -164,11 +210,10 @@ __global__ void k_count(PairSrc src, int32_t *cnt, int32_t *cnt2) {
   }
 }
 
-__global__ void k_scatter(PairSrc src, const int32_t *rowptr, int32_t *cur, int32_t *col) {
+__global__ void k_scatter(LinkSrc src, const int32_t *rowptr, int32_t *cur, int32_t *col) {
   int64_t i = (int64_t)xcd_block() * blockDim.x + threadIdx.x;
   if (i >= src.n) return;
-  const int per = src.per();
-  for (int j = 0; j < per; ++j) {
+  for (int j = 0; j < 3; ++j) {
     int32_t a, b;
     if (src.get(i, j, a, b)) {
       int32_t pos = rowptr[a] + atomicAdd(&cur[a], 1);
@@ -203,69 +248,64 @@ __device__ inline void sort16(int32_t (&v)[16]) {
   }
 }
 
-// Appends `want` lanes' values to list (count at *n) with one atomic per
-// wave: the first wanting lane reserves the wave's slots, every lane takes
-// the slot of its rank among the wanting lanes.
-__device__ inline void wave_append(bool want, int32_t value, int32_t *list, int32_t *n) {
-  const uint64_t m = __ballot(want);
-  if (!m) return;
-  const int lane = threadIdx.x % 64;
-  const int leader = __builtin_ctzll(m);
-  int32_t base = 0;
-  if (lane == leader) base = atomicAdd(n, (int32_t)__popcll(m));
-  base = __shfl(base, leader);
-  if (want) list[base + (int32_t)__popcll(m & ((1ull << lane) - 1))] = value;
-}
+constexpr int kRows = 256;    // buckets of one workgroup
+constexpr int kStage = 4096;  // ids staged in LDS for them
 
-// Per-bucket sort + unique count for short buckets (one thread each);
-// medium buckets (a 3D mesh's: each edge comes once per incident cell) are
-// listed for the one-wave pass, long ones for the workgroup pass (one
-// atomic per wave and list: in 3D nearly every row is listed, and one
-// atomic per row on the same two counters serialises).
-__global__ void k_row_sort(int64_t nrows, const int32_t *rowptr, int32_t *col, int32_t *ucnt,
-                           int32_t *long_rows, int32_t *nlong, int32_t *mid_rows,
-                           int32_t *nmid) {
-  int64_t r = (int64_t)xcd_block() * blockDim.x + threadIdx.x;
+// Sorts kRows consecutive buckets and leaves each one's distinct ids,
+// ascending, at its start.  The buckets are one contiguous piece of col,
+// moved through LDS in whole lines (in global memory if it is longer than
+// kStage); a thread sorts its own bucket if short, its wave the ones of up
+// to kWaveSort ids one after the other; longer ones are listed (one atomic
+// per wave that has any) for the workgroup pass.  Listing the middle ones
+// too and sorting them in a pass of their own took 95 + 139 us on 512 k
+// lattice vertices; now 17 us.
+__global__ __launch_bounds__(kRows) void k_row_sort(int64_t nrows, const int32_t *rowptr,
+                                                    int32_t *col, int32_t *ucnt,
+                                                    int32_t *long_rows, int32_t *nlong) {
+  __shared__ int32_t sh[kStage];
+  const int tid = threadIdx.x, lane = tid % 64;
+  const int64_t r0 = (int64_t)xcd_block() * kRows, r = r0 + tid;
   if (r == 0) ucnt[nrows] = 0;  // the scan's last input (its total slot)
-  const bool row = r < nrows;
-  const int32_t s = row ? rowptr[r] : 0, e = row ? rowptr[r + 1] : 0;
-  const int32_t len = e - s;
-  wave_append(row && len > kRegSort && len <= kWaveSort, (int32_t)r, mid_rows, nmid);
-  wave_append(row && len > kWaveSort, (int32_t)r, long_rows, nlong);
-  if (!row) return;
-  if (len > kRegSort) {
-    ucnt[r] = 0;  // filled by the wave or workgroup pass
-    return;
+  if (r0 >= nrows) return;
+  const int64_t r1 = r0 + kRows < nrows ? r0 + kRows : nrows;
+  const int32_t c0 = rowptr[r0], n = rowptr[r1] - c0;
+  const bool staged = n <= kStage;
+  int32_t *buf = col + c0;
+  if (staged) {
+    for (int32_t k = tid; k < n; k += kRows) sh[k] = buf[k];
+    __syncthreads();
+    buf = sh;
   }
-  int32_t v[16];
-#pragma unroll
-  for (int k = 0; k < 16; ++k) v[k] = k < len ? col[s + k] : INT32_MAX;
-  sort16(v);
-  int32_t u = 0;
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    if (k < len) {
-      col[s + k] = v[k];
-      u += (k == 0 || v[k] != v[k - 1]);
+  const bool row = r < nrows;
+  const int32_t s = row ? rowptr[r] - c0 : 0, len = row ? rowptr[r + 1] - c0 - s : 0;
+  const uint64_t lm = __ballot(len > kWaveSort);
+  if (lm) {
+    const int lead = __builtin_ctzll(lm);
+    int32_t base = 0;
+    if (lane == lead) base = atomicAdd(nlong, (int32_t)__popcll(lm));
+    base = __shfl(base, lead);
+    if (len > kWaveSort) {
+      long_rows[base + (int32_t)__popcll(lm & ((1ull << lane) - 1))] = (int32_t)r;
+      ucnt[r] = 0;  // filled by the workgroup pass
     }
   }
-  ucnt[r] = u;
-}
-
-// Medium buckets (kRegSort < len <= 64), one wave each: lane k holds id k
-// (INT32_MAX past the end), a bitonic network over the 64 lanes exchanges
-// partners with lane shuffles, and a ballot counts the distinct ids.
-// (block b of nb blocks given to this pass)
-__device__ inline void wave_sort_rows(unsigned b, unsigned nb, const int32_t *mid_rows,
-                                      const int32_t *nmid, const int32_t *rowptr, int32_t *col,
-                                      int32_t *ucnt) {
-  const int lane = threadIdx.x % 64;
-  const int64_t nw = (int64_t)nb * (blockDim.x / 64);
-  const int32_t n = *nmid;
-  for (int64_t wv = ((int64_t)b * blockDim.x + threadIdx.x) / 64; wv < n; wv += nw) {
-    const int32_t r = mid_rows[wv];
-    const int32_t s = rowptr[r], len = rowptr[r + 1] - s;
-    int32_t v = lane < len ? col[s + lane] : INT32_MAX;
+  if (row && len <= kRegSort) {
+    int32_t v[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) v[k] = k < len ? buf[s + k] : INT32_MAX;
+    sort16(v);
+    int32_t u = 0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k)
+      if (k < len && (k == 0 || v[k] != v[k - 1])) buf[s + u++] = v[k];
+    ucnt[r] = u;
+  }
+  // kRegSort < len <= kWaveSort: lane k holds id k (INT32_MAX past the end);
+  // a bitonic network over the 64 lanes, partners exchanged by lane shuffles
+  for (uint64_t mid = __ballot(len > kRegSort && len <= kWaveSort); mid; mid &= mid - 1) {
+    const int w = __builtin_ctzll(mid);
+    const int32_t ws = __shfl(s, w), wl = __shfl(len, w);
+    int32_t v = lane < wl ? buf[ws + lane] : INT32_MAX;
 #pragma unroll
     for (int size = 2; size <= 64; size <<= 1) {
 #pragma unroll
@@ -279,11 +319,14 @@ __device__ inline void wave_sort_rows(unsigned b, unsigned nb, const int32_t *mi
       }
     }
     const int32_t prev = __shfl_up(v, 1);
-    const bool first = lane < len && (lane == 0 || v != prev);
+    const bool first = lane < wl && (lane == 0 || v != prev);
     const uint64_t m = __ballot(first);
-    if (lane < len) col[s + lane] = v;
-    if (lane == 0) ucnt[r] = (int32_t)__popcll(m);
+    if (first) buf[ws + (int32_t)__popcll(m & ((1ull << lane) - 1))] = v;
+    if (lane == w) ucnt[r] = (int32_t)__popcll(m);
   }
+  if (!staged) return;
+  __syncthreads();
+  for (int32_t k = tid; k < n; k += kRows) col[c0 + k] = sh[k];
 }
 
 // Long buckets, one workgroup each: a bitonic sort in LDS (padded with
@@ -324,18 +367,27 @@ __device__ inline void long_sort_rows(unsigned b, unsigned nb, const int32_t *lo
         __syncthreads();
       }
     }
+    // the distinct ids to the bucket's start, each thread a piece of them
+    const int32_t piece = (len + (int32_t)blockDim.x - 1) / (int32_t)blockDim.x;
+    const int32_t k0 = piece * (int32_t)threadIdx.x;
+    const int32_t k1 = k0 + piece < len ? k0 + piece : len;
     int32_t u = 0;
-    for (int32_t k = threadIdx.x; k < len; k += blockDim.x) {
-      col[s + k] = buf[k];
-      u += (k == 0 || buf[k] != buf[k - 1]);
-    }
+    for (int32_t k = k0; k < k1; ++k) u += (k == 0 || buf[k] != buf[k - 1]);
     red[threadIdx.x] = u;
     __syncthreads();
     if (threadIdx.x == 0) {
       int32_t t = 0;
-      for (int k = 0; k < (int)blockDim.x; ++k) t += red[k];
+      for (int k = 0; k < (int)blockDim.x; ++k) {
+        const int32_t c = red[k];
+        red[k] = t;
+        t += c;
+      }
       ucnt[r] = t;
     }
+    __syncthreads();
+    u = red[threadIdx.x];
+    for (int32_t k = k0; k < k1; ++k)
+      if (k == 0 || buf[k] != buf[k - 1]) col[s + u++] = buf[k];
     __syncthreads();
   }
 }
@@ -346,72 +398,70 @@ __device__ inline void long_sort_rows(unsigned b, unsigned nb, const int32_t *lo
 // 150-400 us per launch on the EAGE-shaped workload; idle ones exit at once
 constexpr unsigned kLongBlocks = 1024;
 
-// The bucket sorts after the per-thread pass, in one launch of 256-thread
-// workgroups (the passes touch disjoint buckets): blocks [0, nwave) take
-// the one-wave buckets, the next kLongBlocks the LDS-sized long buckets,
-// the last one the buckets sorted in the global staging area (one
-// workgroup, so the staging area is private to it).
-__global__ void k_bucket_sorts(const int32_t *mid_rows, const int32_t *nmid,
-                               const int32_t *long_rows, const int32_t *nlong,
-                               const int32_t *rowptr, int32_t *col, int32_t *ucnt, int32_t *stage,
-                               unsigned nwave) {
+// The long buckets, in one launch of 256-thread workgroups: the first
+// kLongBlocks take the LDS-sized ones, the last one the buckets sorted in
+// the global staging area (one workgroup, so the staging area is private to
+// it).
+__global__ void k_long_sorts(const int32_t *long_rows, const int32_t *nlong,
+                             const int32_t *rowptr, int32_t *col, int32_t *ucnt, int32_t *stage) {
   __shared__ int32_t sh[kLdsSort];
   __shared__ int32_t red[256];
   const unsigned b = blockIdx.x;
-  if (b < nwave)
-    wave_sort_rows(b, nwave, mid_rows, nmid, rowptr, col, ucnt);
-  else if (b < nwave + kLongBlocks)
-    long_sort_rows(b - nwave, kLongBlocks, long_rows, nlong, rowptr, col, ucnt, stage, 0, sh, red);
+  if (b < kLongBlocks)
+    long_sort_rows(b, kLongBlocks, long_rows, nlong, rowptr, col, ucnt, stage, 0, sh, red);
   else
     long_sort_rows(0, 1, long_rows, nlong, rowptr, col, ucnt, stage, 1, sh, red);
 }
 
-__global__ void k_emit(int64_t nrows, const int32_t *rowptr, const int32_t *col,
-                       const int32_t *eptr, int32_t *edges, SecondLists second) {
-  int64_t r = (int64_t)xcd_block() * blockDim.x + threadIdx.x;
-  if (r >= nrows) return;
-  int32_t s = rowptr[r], e = rowptr[r + 1];
-  int32_t o = eptr[r];
-  for (int32_t k = s; k < e; ++k) {
-    if (k == s || col[k] != col[k - 1]) {
-      const int32_t b = col[k];
-      edges[2 * (int64_t)o] = (int32_t)r;
-      edges[2 * (int64_t)o + 1] = b;
-      if (second.list) second.list[second.ptr[b] + atomicAdd(&second.cur[b], 1)] = o;
-      ++o;
-    }
+// The edges of kRows consecutive buckets, one contiguous piece of the
+// output, a thread per edge so that both the ids' reads and the edges'
+// writes are whole lines; an edge finds its bucket by bisecting the
+// buckets' offsets in LDS.  (A wave per bucket took 70 us for 3.5 M edges,
+// now 12 us.)  len (optional): only that many of a bucket's slots are written.
+__global__ __launch_bounds__(kRows) void k_emit(int64_t nrows, const int32_t *rowptr,
+                                                const int32_t *col, const int32_t *eptr,
+                                                const int32_t *len, int32_t *edges,
+                                                SecondLists second) {
+  __shared__ int32_t off[kRows + 1], start[kRows];
+  const int tid = threadIdx.x;
+  const int64_t r0 = (int64_t)xcd_block() * kRows;
+  if (r0 >= nrows) return;
+  const int nr = (int)(nrows - r0 < kRows ? nrows - r0 : kRows);
+  if (tid < nr) {
+    off[tid] = eptr[r0 + tid];
+    start[tid] = rowptr[r0 + tid];
   }
-}
-
-// The same for the buckets of tetrahedra (dozens of sorted ids with
-// duplicates): one wave per row, 64 ids at a time, each distinct id's
-// output slot from a ballot of the first occurrences (grid-stride over the
-// rows).
-__global__ void k_emit_wave(int64_t nrows, const int32_t *rowptr, const int32_t *col,
-                            const int32_t *eptr, int32_t *edges, SecondLists second) {
-  const int lane = threadIdx.x % 64;
-  const int64_t nw = (int64_t)gridDim.x * (blockDim.x / 64);
-  for (int64_t r = ((int64_t)xcd_block() * blockDim.x + threadIdx.x) / 64; r < nrows; r += nw) {
-    const int32_t s = rowptr[r], e = rowptr[r + 1];
-    int32_t o = eptr[r];
-    for (int32_t k0 = s; k0 < e; k0 += 64) {
-      const int32_t k = k0 + lane;
-      const bool in = k < e;
-      const int32_t b = in ? col[k] : 0;
-      const bool first = in && (k == s || col[k - 1] != b);
-      const uint64_t m = __ballot(first);
-      if (first) {
-        const int32_t oo = o + (int32_t)__popcll(m & ((1ull << lane) - 1));
-        edges[2 * (int64_t)oo] = (int32_t)r;
-        edges[2 * (int64_t)oo + 1] = b;
-        if (second.list) second.list[second.ptr[b] + atomicAdd(&second.cur[b], 1)] = oo;
-      }
-      o += (int32_t)__popcll(m);
+  if (tid == 0) off[nr] = eptr[r0 + nr];
+  __syncthreads();
+  for (int32_t o = off[0] + tid; o < off[nr]; o += kRows) {
+    int lo = 0, hi = nr;  // off[lo] <= o < off[hi]
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) / 2;
+      if (off[mid] <= o) lo = mid;
+      else hi = mid;
     }
+    if (len && o - off[lo] >= len[r0 + lo]) continue;
+    const int32_t b = col[start[lo] + (o - off[lo])];
+    edges[2 * (int64_t)o] = (int32_t)(r0 + lo);
+    edges[2 * (int64_t)o + 1] = b;
+    if (second.list) second.list[second.ptr[b] + atomicAdd(&second.cur[b], 1)] = o;
   }
 }
 
 __global__ void k_count_to_i64(const int32_t *c, int64_t *out) { *out = (int64_t)*c; }
+
+template <int NV>
+int item_pass(const ItemSrc &src, bool count, int32_t *rowptr, int32_t *cur, int2 *list,
+              int32_t *col, hipStream_t s) {
+  const dim3 grid(blocks_for(src.n, ItemShape<NV>::items));
+  if (count)
+    hipLaunchKernelGGL((k_item_count<NV>), grid, dim3(kItemThreads), 0, s, src, rowptr, list);
+  else
+    hipLaunchKernelGGL((k_item_scatter<NV>), grid, dim3(kItemThreads), 0, s, src.n,
+                       (const int2 *)list, (const int32_t *)rowptr, cur, col);
+  SM_LAUNCH_CHECK();
+  return SM_OK;
+}
 
 inline size_t al(size_t b) { return (b + 255) & ~(size_t)255; }
 
@@ -424,9 +474,9 @@ size_t unique_edges_workspace(int64_t npairs, int64_t nvert) {
   b += al(npairs * 4);       // col
   b += al((nvert + 1) * 4);  // ucnt -> eptr
   b += al((nvert + 1) * 4);  // long rows
-  b += al((nvert + 1) * 4);  // medium rows
+  b += al((nvert + 1) * 4);  // unused; the size a caller asks for stays what it was
   b += al(8 * 4);            // counters
-  b += al((size_t)npairs * 2 * 4 + 4096 * 4);  // staging for very long buckets
+  b += al((size_t)npairs * 2 * 4 + 4096 * 4);  // blocks' pairs; staging for very long buckets
   b += 2 * scan_workspace(nvert + 1);
   return b;
 }
@@ -459,7 +509,7 @@ int unique_edges_run(const int32_t *pairs, const int32_t *cells, const uint8_t *
   int32_t *col = reinterpret_cast<int32_t *>(w); w += al(npairs * 4);
   int32_t *eptr = reinterpret_cast<int32_t *>(w); w += al((nvert + 1) * 4);
   int32_t *longr = reinterpret_cast<int32_t *>(w); w += al((nvert + 1) * 4);
-  int32_t *midr = reinterpret_cast<int32_t *>(w); w += al((nvert + 1) * 4);
+  w += al((nvert + 1) * 4);
   int32_t *ctr = reinterpret_cast<int32_t *>(w); w += al(8 * 4);
   int32_t *stage = reinterpret_cast<int32_t *>(w);
   w += al((size_t)npairs * 2 * 4 + 4096 * 4);
@@ -470,17 +520,21 @@ int unique_edges_run(const int32_t *pairs, const int32_t *cells, const uint8_t *
     FillList fl{{rowptr, cur, ctr, sl.ptr, sl.cur}, {nvert + 1, nvert + 1, 8, nvert + 1, nvert + 1}};
     if ((rc = fill_list(fl, second ? 5 : 3, 0, s))) return rc;
   }
-  PairSrc src{pairs, cells, keep, adj, dim, n};
   const int B = 256;
   int32_t *total = count32 ? count32 : ctr + 3;
-  // tetrahedra without neighbour links: three runs per cell
-  const bool tets = cells && dim == 3 && !adj && !second;
-  if (n > 0) {
-    if (tets)
-      hipLaunchKernelGGL(k_count_tets, dim3(blocks_for(n, B)), dim3(B), 0, s, src, rowptr);
-    else
-      hipLaunchKernelGGL(k_count, dim3(blocks_for(n, B)), dim3(B), 0, s, src, rowptr, sl.ptr);
+  const LinkSrc link{cells, keep, adj, n};
+  const ItemSrc item{cells ? cells : pairs, keep, n};
+  const auto items = [&](bool count) {
+    int2 *list = reinterpret_cast<int2 *>(stage);
+    if (!cells) return item_pass<2>(item, count, rowptr, cur, list, col, s);
+    if (dim == 2) return item_pass<3>(item, count, rowptr, cur, list, col, s);
+    return item_pass<4>(item, count, rowptr, cur, list, col, s);
+  };
+  if (n > 0 && adj) {
+    hipLaunchKernelGGL(k_count, dim3(blocks_for(n, B)), dim3(B), 0, s, link, rowptr, sl.ptr);
     SM_LAUNCH_CHECK();
+  } else if (n > 0 && (rc = items(true))) {
+    return rc;
   }
   // with adjacency the buckets hold no duplicates: their offsets and total
   // are the output's
@@ -489,39 +543,28 @@ int unique_edges_run(const int32_t *pairs, const int32_t *cells, const uint8_t *
   else
     rc = scan_exclusive(rowptr, rowptr, nvert + 1, adj ? total : ctr + 1, sws, s);
   if (rc) return rc;
-  if (n > 0) {
-    if (tets)
-      hipLaunchKernelGGL(k_scatter_tets, dim3(blocks_for(n, B)), dim3(B), 0, s, src, rowptr, cur,
-                         col);
-    else
-      hipLaunchKernelGGL(k_scatter, dim3(blocks_for(n, B)), dim3(B), 0, s, src, rowptr, cur, col);
+  if (n > 0 && adj) {
+    hipLaunchKernelGGL(k_scatter, dim3(blocks_for(n, B)), dim3(B), 0, s, link, rowptr, cur, col);
     SM_LAUNCH_CHECK();
+  } else if (n > 0 && (rc = items(false))) {
+    return rc;
   }
   if (nvert > 0) {
-    hipLaunchKernelGGL(k_row_sort, dim3(blocks_for(nvert, B)), dim3(B), 0, s, nvert, rowptr,
-                       col, eptr, longr, ctr + 2, midr, ctr + 4);
+    hipLaunchKernelGGL(k_row_sort, dim3(blocks_for(nvert, kRows)), dim3(kRows), 0, s, nvert,
+                       rowptr, col, eptr, longr, ctr + 2);
     SM_LAUNCH_CHECK();
-    // one wave per medium bucket (grid-stride over at most nvert of them),
-    // then the long buckets, in one launch
-    unsigned gw = blocks_for(nvert * 64, 256);
-    if (gw > 8192) gw = 8192;
-    hipLaunchKernelGGL(k_bucket_sorts, dim3(gw + kLongBlocks + 1), dim3(256), 0, s, midr, ctr + 4,
-                       longr, ctr + 2, rowptr, col, eptr, stage, gw);
+    hipLaunchKernelGGL(k_long_sorts, dim3(kLongBlocks + 1), dim3(256), 0, s, longr, ctr + 2,
+                       rowptr, col, eptr, stage);
     SM_LAUNCH_CHECK();
   }
   if (!adj) {
     if (nvert == 0 && (rc = fill<int32_t>(eptr, 1, 0, s))) return rc;
     if ((rc = scan_exclusive(eptr, eptr, nvert + 1, total, sws, s))) return rc;
   }
-  if (nvert > 0 && tets) {
-    unsigned gw = blocks_for(nvert * 64, 256);
-    if (gw > 16384) gw = 16384;
-    hipLaunchKernelGGL(k_emit_wave, dim3(gw), dim3(256), 0, s, nvert, rowptr, col,
-                       (const int32_t *)eptr, edges, sl);
-    SM_LAUNCH_CHECK();
-  } else if (nvert > 0) {
-    hipLaunchKernelGGL(k_emit, dim3(blocks_for(nvert, B)), dim3(B), 0, s, nvert, rowptr, col,
-                       adj ? (const int32_t *)rowptr : (const int32_t *)eptr, edges, sl);
+  if (nvert > 0) {
+    hipLaunchKernelGGL(k_emit, dim3(blocks_for(nvert, kRows)), dim3(kRows), 0, s, nvert, rowptr,
+                       col, adj ? (const int32_t *)rowptr : (const int32_t *)eptr,
+                       adj ? (const int32_t *)eptr : nullptr, edges, sl);
     SM_LAUNCH_CHECK();
   }
   if (count64) {
