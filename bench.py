@@ -6,14 +6,15 @@ Workload (default): the 3D many-primitive CSG of seismicmesh_amd.workloads
 3) at uniform h = 0.015 (~0.5 M vertices).  Two paths run the same
 iterations from the same initial points:
 
-* fused: the tetrahedralisation built by 16 host threads inserting the
-  points of 16 slabs into one shared tetrahedralisation, its cells sorted
-  into pinned memory and copied to the device in pieces, and a neural SDF
-  surrogate (3 -> 256 x4 -> 1, BF16 matrix-core inference) trained here by
-  the library's own kernels on 4 M samples of the exact SDF deciding the
+* fused: the tetrahedralisation found on the device (what it leaves to the
+  host, such as the degenerate initial lattice, by 16 host threads inserting
+  the points of 16 slabs into one shared tetrahedralisation), and a neural
+  SDF surrogate (3 -> 256 x4 -> 1, BF16 matrix-core inference) trained here
+  by the library's own kernels on 4 M samples of the exact SDF deciding the
   centroid filter and the projection test away from the boundary (exact
   SDF inside the band);
-* plain: the serial tetrahedralisation and the exact SDF everywhere.
+* plain: the same with one host thread for what is left to the host, and
+  the exact SDF everywhere.
 
 A step is one force iteration over the whole point set: re-triangulation,
 centroid filter, sorted unique edges, bar forces, gather, update and Newton
@@ -300,10 +301,10 @@ def mlp_measure(npts=1 << 22, reps=10):
 
 
 def bench_3d(args):
-    """The 3D workloads: the fused path (slab-parallel tetrahedralisation
-    overlapped with the device filter, and for the CSG a trained surrogate)
-    against the plain path (serial tetrahedralisation, exact SDF), same
-    points, same iterations."""
+    """The 3D workloads: the fused path (device tetrahedralisation, host
+    builds slab-parallel and overlapped with the device filter, and for the
+    CSG a trained surrogate) against the plain path (host builds serial,
+    exact SDF), same points, same iterations."""
     import torch
     from seismicmesh_amd import generation, workloads
     from seismicmesh_amd import mesh_utils as mu
@@ -497,16 +498,17 @@ def bench_3d(args):
         "data": "synthetic",
         "config": dict(
             wl, N=N, edges=E, cells=C,
-            path=("tetrahedralisation by %d host threads inserting the points of %d slabs "
-                  "(axis %d) into one shared tetrahedralisation, its cells sorted into pinned "
-                  "memory and copied to the device piece by piece; device filter, edges, "
+            path=("tetrahedralisation on the device, one wave per vertex star (builds it "
+                  "leaves to the host: %d threads inserting the points of %d slabs along axis "
+                  "%d into one shared tetrahedralisation); device filter, edges, "
                   "forces, update, projection%s"
                   % (threads, args.slabs, axis,
                      "; surrogate-steered filter and projection (exact SDF in the band)"
                      if neural else "")),
             plain_value=round(plain_value, 1),
             speedup_vs_plain=round(value / plain_value, 3),
-            plain_path="serial tetrahedralisation, exact SDF, same device kernels",
+            plain_path="the same tetrahedralisation (builds left to the host: one thread), "
+                       "exact SDF, same device kernels",
             points_identical_to_plain=identical,
             min_quality=stats["min_quality"], plain_min_quality=plain_stats["min_quality"],
             p1_quality=stats["p1_quality"], plain_p1_quality=plain_stats["p1_quality"],
@@ -738,7 +740,7 @@ def main():
         "data": "synthetic",
         "config": dict(wl, N=N, edges=E, cells=C,
                        path=("device flips; one captured graph launch per iteration"
-                             if dim == 2 else "host tetrahedralisation, device filter, edges, "
+                             if dim == 2 else "device tetrahedralisation, filter, edges, "
                              "forces, update and projection"),
                        plain_value=round(N * args.steps / plain_elapsed, 1),
                        plain_path="same kernels launched one by one, host sync per stage",
