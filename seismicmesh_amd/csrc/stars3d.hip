@@ -1084,10 +1084,15 @@ __global__ __launch_bounds__(64 * kStarWaves, EXACT ? 1 : (FAR ? 3 : 4)) void k_
     int64_t n, const StarGrid *gp, const SPt *ps, const int32_t *start, const Node *nodes,
     const int32_t *list, const int32_t *nlist, int32_t most, int32_t *far, int32_t *exact,
     int32_t *hubs, int32_t *pool, int64_t pool_cap, int32_t *poff, int32_t *pcnt,
-    int32_t *rowcnt, int32_t *status) {
+    int32_t *rowcnt, int32_t *status, int32_t most_exact) {
   __shared__ StarLds shm[kStarWaves];
   __shared__ FarLds fshm[FAR ? kStarWaves : 1];
   if (status[kStFail]) return;
+  // too many uncertain stars after the near pass: the rest is no use
+  if (FAR && status[kStX] > most_exact) {
+    if (threadIdx.x == 0) status[kStFail] = 5;
+    return;
+  }
   const int lane = threadIdx.x % 64;
   const int64_t items = list ? (int64_t)*nlist : n;
   if (list && items > most) {
@@ -1098,6 +1103,9 @@ __global__ __launch_bounds__(64 * kStarWaves, EXACT ? 1 : (FAR ? 3 : 4)) void k_
   const unsigned blk = list ? blockIdx.x : xcd_block();
   const int wv = uni(threadIdx.x / 64);
   for (int64_t w = (int64_t)blk * kStarWaves + wv; w < items; w += nw) {
+    if (EXACT &&
+        __hip_atomic_load(&status[kStFail], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      return;
     const int self = uni(list ? list[w] : (int)w);
     const SPt q = ps[self];
     const int32_t id = uni(q.id);
@@ -1397,18 +1405,25 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
                        dim3(B), 0, s, g, l, start, ps, nodes);
   }
   // uncertain predicates beyond this many vertices: a degenerate lattice,
-  // which the host settles sooner
-  const int32_t most_exact = (int32_t)std::max<int64_t>(1024, n / 32);
+  // which the host settles sooner.  An exact star takes 0.25 us when the
+  // chip is full of them: 523 k points of the 76-primitive solid, two to
+  // eleven moves after their lattice, take 103 ms with 282 k exact stars, 91
+  // with 222 k, 54 with 36 k, against 105-130 ms on 16 host threads whatever
+  // they hold (119 with 344 k: even).  Few stars do not fill the chip, and
+  // the longest chain decides: 3 k points 23 ms with 2.7 k exact stars, the
+  // host's one thread 9.
+  const int32_t most_exact =
+      (int32_t)(n >= 65536 ? n / 2 : std::max<int64_t>(1024, n / 32));
   constexpr int W = kStarWaves;
   hipLaunchKernelGGL((k_stars<false, false>), dim3(blocks_for(n, W)), dim3(64 * W), 0, s, n, g, ps,
                      start, nodes, (const int32_t *)nullptr, (const int32_t *)nullptr, 0, lf, lx,
-                     hub, pool, pool_cap, poff, pcnt, row, st);
+                     hub, pool, pool_cap, poff, pcnt, row, st, most_exact);
   hipLaunchKernelGGL((k_stars<true, false>), dim3(blocks_for(n, 4 * W)), dim3(64 * W), 0, s, n, g,
                      ps, start, nodes, lf, st + kStF, (int32_t)n, lf, lx, hub, pool, pool_cap,
-                     poff, pcnt, row, st);
+                     poff, pcnt, row, st, most_exact);
   hipLaunchKernelGGL((k_stars<true, true>), dim3((unsigned)std::min<int64_t>(1024, gn)),
                      dim3(64 * W), 0, s, n, g, ps, start, nodes, lx, st + kStX, most_exact, lf, lx,
-                     hub, pool, pool_cap, poff, pcnt, row, st);
+                     hub, pool, pool_cap, poff, pcnt, row, st, most_exact);
   SM_LAUNCH_CHECK();
   const auto place = [&]() -> int {
     if ((rc = fill<int32_t>(row + n, 1, 0, s))) return rc;
@@ -1423,7 +1438,10 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
   if ((rc = place())) return rc;
   const int32_t *hs = sc->h_status;
   const auto leave = [&]() {
-    sc->skip = 3;  // what fails now (a degenerate lattice) likely fails again
+    // what fails now (a degenerate lattice) likely fails again; but a large
+    // one is known for it early (5 of 130 ms) and loses a share of its
+    // uncertain stars with every move
+    sc->skip = sc->h_status[kStFail] == 5 && n >= 65536 ? 2 : 3;
     return SM_OK;
   };
   if (hs[kStFail] || hs[kStHub] > kMaxHubs || hs[kStTotal] < 0) return leave();

@@ -123,3 +123,21 @@ def test_a_failed_build_is_followed_by_the_host_then_the_device_again():
         assert np.array_equal(m.cells(), _host(np.ascontiguousarray(p)))
     assert m.stats()["parallel_builds"] >= 2
     m.close()
+
+
+@pytest.mark.parametrize("side,share,by_device", [(40, 0.3, False), (41, 0.3, True),
+                                                  (41, 0.7, False)])
+def test_lattice_share_left_to_the_host(side, share, by_device):
+    # exact cubes in part of the box (their stars take the exact pass), a
+    # jittered lattice in the rest: from 65536 points on (41^3) the device
+    # settles up to half of the vertices exactly, below that 1 in 32.
+    # Coordinates in [1, 2): one binary exponent, the exact stage's range
+    rng = np.random.default_rng(side)
+    g = 1.0 + np.arange(side) / 64.0
+    p = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+    moved = p[:, 0] > 1.0 + share * side / 64.0
+    p[moved] += rng.uniform(0.0, 0.2 / 64.0, (int(moved.sum()), 3))
+    p = np.ascontiguousarray(p)
+    cells, dev = _device(p, 1 / 64)
+    assert dev == by_device
+    assert np.array_equal(cells, _host(p))
