@@ -47,8 +47,8 @@ HBM_PEAK_GBS = 8000.0
 # kernels timed alone by the handle's event profiler, by phase name
 SINGLE_KERNEL = {"centroid_filter": "k_keep", "edge_geom": "k_edge_geom",
                  "edge_force": "k_edge_force", "vertex_update": "k_vertex_update",
-                 "flip_mark": "k_mark", "unique_edges": "edge build (k_count, scan, "
-                 "k_scatter, k_bucket_sorts, k_emit)"}
+                 "flip_mark": "k_mark", "unique_edges": "edge build (counts, scans, "
+                 "scatter, k_row_sort, k_long_sorts, k_emit)"}
 
 
 def cpu_info():
