@@ -365,6 +365,11 @@ int sm_mesher_stats(sm_mesher *m, int64_t *stats, int nstats);
  * Replaces the per-rank slabs of mesh_generator.py:808-852, :867-877 and
  * decomp/blocker.py:4-111 (axis as the reference's `axis` option). */
 int sm_mesher_set_slabs(sm_mesher *m, int axis, int nslabs, int nthreads);
+/* 3D handles: the most device memory the tetrahedralisation may take for
+ * scratch (about 0.6 kB a point); builds that need more, and those for which
+ * the device has no room, are made on the host: the same cells.  0: no limit
+ * of its own (the default). */
+int sm_mesher_set_scratch_limit(sm_mesher *m, int64_t bytes);
 /* Per-phase kernel timing with HIP events recorded on the handle's stream.
  * Phases: 0 flip rounds, 1 centroid filter, 2 unique edges + edge lists,
  * 3 bar lengths and sizing, 4 L0 sums, 5 bar forces, 6 gather + update +

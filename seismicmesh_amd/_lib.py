@@ -123,6 +123,7 @@ _PROTOS = {
     "sm_mesher_get_triangulation": (_i64, [_vp, _vp, _vp, _i64]),
     "sm_mesher_stats": (_int, [_vp, _vp, _int]),
     "sm_mesher_set_slabs": (_int, [_vp, _int, _int, _int]),
+    "sm_mesher_set_scratch_limit": (_int, [_vp, _i64]),
     "sm_mesher_set_graph": (_int, [_vp, _int]),
     "sm_mesher_profile": (_int, [_vp, _int]),
     "sm_mesher_profile_read": (_int, [_vp, _vp, _vp, _int]),

@@ -852,6 +852,14 @@ extern "C" int sm_mesher_stats(sm_mesher *m, int64_t *stats, int nstats) {
   return SM_OK;
 }
 
+extern "C" int sm_mesher_set_scratch_limit(sm_mesher *m, int64_t bytes) {
+  SM_CHECK(m && bytes >= 0, SM_ERR_ARG, "mesher_set_scratch_limit: bad argument");
+  SM_CHECK(m->dim == 3, SM_ERR_ARG, "mesher_set_scratch_limit: 3D handles only");
+  m->stars.max_bytes = bytes == 0 ? SIZE_MAX : (size_t)bytes;
+  m->stars.skip = 0;
+  return SM_OK;
+}
+
 extern "C" int sm_mesher_set_slabs(sm_mesher *m, int axis, int nslabs, int nthreads) {
   SM_CHECK(m, SM_ERR_ARG, "mesher_set_slabs: null handle");
   SM_CHECK(m->dim == 3, SM_ERR_ARG, "mesher_set_slabs: slabs split the 3D tetrahedralisation");

@@ -9,11 +9,12 @@
 
 namespace smk {
 
-// Scratch of the device build (one per handle, sized for its points).
+// Scratch of the device build (one per handle, grown to its largest point
+// set: about 0.6 kB a point).
 struct StarScratch {
-  int64_t cap_n = 0;
   void *mem = nullptr;
   size_t bytes = 0;
+  size_t max_bytes = SIZE_MAX;  // builds that need more go to the host
   int32_t *h_status = nullptr;  // pinned
   int skip = 0;                 // builds left to the host after a failed one
   int64_t builds = 0, hubs = 0;
@@ -33,8 +34,9 @@ constexpr int64_t kStarMinPoints = 512;
 // points (any positive value is correct; it sizes the search grid).
 // Synchronises the stream.  *done is false when the device leaves the build
 // to the host (too few points, points in one plane, predicates its exact
-// stage cannot settle, too many uncertain ones or very large stars); nothing is
-// written then that the host build does not replace.
+// stage cannot settle, too many uncertain ones or very large stars, no memory
+// for the scratch); nothing is written then that the host build does not
+// replace.
 int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacing, int32_t *tet,
                       int64_t cap, int64_t *count, bool *done, hipStream_t s);
 

@@ -45,6 +45,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <new>
 #include <vector>
 
 #include "common.h"
@@ -1327,7 +1328,7 @@ void stars_free(StarScratch *s) {
   if (s->h_status) (void)hipHostFree(s->h_status);
   s->mem = nullptr;
   s->h_status = nullptr;
-  s->cap_n = 0;
+  s->bytes = 0;
 }
 
 int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacing, int32_t *tet,
@@ -1358,17 +1359,29 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
   const size_t o_row = take((size_t)(n + 1) * 4), o_rowp = take((size_t)(n + 1) * 4);
   const size_t o_pool = take((size_t)pool_cap * 12);
   const size_t o_ws = take(scan_workspace(std::max(cells, n) + 1));
-  if (sc->cap_n != n) {
+  // without room for the scratch the host build does it, which needs none
+  // on the device
+  const auto no_room = [&]() {
+    (void)hipGetLastError();
+    sc->skip = 3;
+    return SM_OK;
+  };
+  if (off > sc->max_bytes) return no_room();
+  if (sc->bytes < off) {
     if (sc->mem) (void)hipFree(sc->mem);
     sc->mem = nullptr;
-    sc->cap_n = 0;
-    SM_HIP(hipMalloc(&sc->mem, off));
-    sc->cap_n = n;
+    sc->bytes = 0;
+    if (hipMalloc(&sc->mem, off) != hipSuccess) {
+      sc->mem = nullptr;
+      return no_room();
+    }
     sc->bytes = off;
   }
-  if (!sc->h_status)
-    SM_HIP(hipHostMalloc((void **)&sc->h_status, kStWords * sizeof(int32_t),
-                         hipHostMallocDefault));
+  if (!sc->h_status && hipHostMalloc((void **)&sc->h_status, kStWords * sizeof(int32_t),
+                                     hipHostMallocDefault) != hipSuccess) {
+    sc->h_status = nullptr;
+    return no_room();
+  }
   char *b = reinterpret_cast<char *>(sc->mem);
   uint64_t *bb = reinterpret_cast<uint64_t *>(b + o_bb);
   StarGrid *g = reinterpret_cast<StarGrid *>(b + o_grid);
@@ -1445,12 +1458,19 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
     return SM_OK;
   };
   if (hs[kStFail] || hs[kStHub] > kMaxHubs || hs[kStTotal] < 0) return leave();
-  if (hs[kStHub] > 0) {
-    // hubs: their rows from their neighbours' stars and, for cells of four
-    // hubs, from the hubs' own triangulation, each cell checked against
-    // every point; some thousand cells, ordered on the host
+  // Hubs: their rows from their neighbours' stars and, for cells of four
+  // hubs, from the hubs' own triangulation, each cell checked against every
+  // point; some thousand cells, ordered on the host.  The host arrays outlive
+  // the copies on the stream, also where memory runs out.
+  struct Cell {
+    int32_t v[4];
+  };
+  std::vector<int32_t> hv, hc, own, hb, rows, to, r0;
+  std::vector<double> hp;
+  std::vector<Cell> all;
+  if (hs[kStHub] > 0) try {
     const int nh = hs[kStHub];
-    std::vector<int32_t> hv((size_t)nh);
+    hv.resize((size_t)nh);
     SM_HIP(hipMemcpyAsync(hv.data(), hub, nh * 4, hipMemcpyDeviceToHost, s));
     SM_HIP(hipStreamSynchronize(s));
     std::sort(hv.begin(), hv.end());
@@ -1467,20 +1487,22 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
                        hpts);
     SM_LAUNCH_CHECK();
     int32_t nc = 0;
-    std::vector<double> hp((size_t)nh * 3);
+    hp.resize((size_t)nh * 3);
     SM_HIP(hipMemcpyAsync(&nc, hcount, 4, hipMemcpyDeviceToHost, s));
     SM_HIP(hipMemcpyAsync(hp.data(), hpts, hp.size() * 8, hipMemcpyDeviceToHost, s));
     SM_HIP(hipStreamSynchronize(s));
     if (nc < 0 || nc > hcap) return leave();
-    std::vector<int32_t> hc((size_t)nc * 4);
+    hc.resize((size_t)nc * 4);
     if (nc) SM_HIP(hipMemcpyAsync(hc.data(), hcells, hc.size() * 4, hipMemcpyDeviceToHost, s));
-    std::vector<int32_t> own;
     if (nh >= 4) {
       smdt::DT3 dt;
       rc = dt.run(hp.data(), nh, 0, 1, 1, [&](int, const int32_t *c, int64_t k) {
         for (int64_t i = 0; i < 4 * k; ++i) own.push_back(hv[(size_t)c[i]]);
       });
-      if (rc) return rc;
+      if (rc) {
+        SM_HIP(hipStreamSynchronize(s));
+        return leave();
+      }
     }
     SM_HIP(hipStreamSynchronize(s));
     if (!own.empty()) {
@@ -1492,7 +1514,7 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
       hipLaunchKernelGGL(k_star_check, dim3(blocks_for(no, W)), dim3(64 * W), 0, s, g, ps, start,
                          nodes, dc, no, posn, bad);
       SM_LAUNCH_CHECK();
-      std::vector<int32_t> hb((size_t)no);
+      hb.resize((size_t)no);
       SM_HIP(hipMemcpyAsync(hb.data(), bad, no * 4, hipMemcpyDeviceToHost, s));
       SM_HIP(hipStreamSynchronize(s));
       for (int c = 0; c < no; ++c) {
@@ -1501,10 +1523,7 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
           hc.insert(hc.end(), own.begin() + 4 * (size_t)c, own.begin() + 4 * (size_t)c + 4);
       }
     }
-    struct Cell {
-      int32_t v[4];
-    };
-    std::vector<Cell> all(hc.size() / 4);
+    all.resize(hc.size() / 4);
     for (size_t i = 0; i < all.size(); ++i) {
       std::memcpy(all[i].v, hc.data() + 4 * i, 16);
       smdt::canonical_tet(all[i].v);
@@ -1513,7 +1532,8 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
       return std::lexicographical_compare(x.v, x.v + 4, y.v, y.v + 4);
     });
     // the hubs' rows were empty so far: count, place, fill
-    std::vector<int32_t> rows((size_t)nh, 0), to(all.size());
+    rows.assign((size_t)nh, 0);
+    to.resize(all.size());
     for (const Cell &c : all) {
       const auto it = std::lower_bound(hv.begin(), hv.end(), c.v[0]);
       if (it == hv.end() || *it != c.v[0]) return leave();
@@ -1525,7 +1545,7 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
     if (hs[kStFail] || hs[kStTotal] > cap || hs[kStTotal] < 0) return leave();
     hipLaunchKernelGGL(k_star_read, dim3(blocks_for(nh, B)), dim3(B), 0, s, nh, hub, rowp, tmp);
     SM_LAUNCH_CHECK();
-    std::vector<int32_t> r0((size_t)nh);
+    r0.resize((size_t)nh);
     SM_HIP(hipMemcpyAsync(r0.data(), tmp, nh * 4, hipMemcpyDeviceToHost, s));
     SM_HIP(hipStreamSynchronize(s));
     size_t at = 0;
@@ -1545,6 +1565,9 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
       SM_HIP(hipStreamSynchronize(s));
     }
     sc->hubs += nh;
+  } catch (const std::bad_alloc &) {
+    SM_HIP(hipStreamSynchronize(s));
+    return leave();
   }
   if (hs[kStTotal] > cap) return leave();
   *count = hs[kStTotal];

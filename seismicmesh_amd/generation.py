@@ -378,6 +378,12 @@ class Mesher:
         _lib.check(_lib.lib.sm_mesher_set_slabs(self.h, int(axis), int(nslabs), int(threads)),
                    "sm_mesher_set_slabs")
 
+    def set_scratch_limit(self, nbytes):
+        """3D: the most device memory the tetrahedralisation may take for
+        scratch (0: no limit); builds that need more are made on the host."""
+        _lib.check(_lib.lib.sm_mesher_set_scratch_limit(self.h, int(nbytes)),
+                   "sm_mesher_set_scratch_limit")
+
 
 def _placeholder(dim):
     return (geo.Disk([0.0, 0.0], 1.0) if dim == 2 else geo.Ball([0.0, 0.0, 0.0], 1.0)).tape()

@@ -141,3 +141,19 @@ def test_lattice_share_left_to_the_host(side, share, by_device):
     cells, dev = _device(p, 1 / 64)
     assert dev == by_device
     assert np.array_equal(cells, _host(p))
+
+
+def test_a_build_without_room_for_its_scratch_goes_to_the_host():
+    # 0.6 kB a point: 100 kB are too little for 2000, 10 MB are enough
+    from seismicmesh_amd import generation, geometry as geo
+    p, h = _points("random2000")
+    m = generation.Mesher([geo.Ball([0.0, 0.0, 0.0], 1e7)], generation._Sizing("const", value=h),
+                          h, 0.2, 0.1 * h, 1e-8 * h, 0, precision=32, dim=3)
+    m.set_points(p)
+    ref = _host(np.ascontiguousarray(p))
+    for limit, built in ((100000, 0), (10000000, 1), (100000, 1), (0, 2)):
+        m.set_scratch_limit(limit)
+        m.triangulate()
+        assert np.array_equal(m.cells(), ref)
+        assert m.stats()["parallel_builds"] == built
+    m.close()
