@@ -515,9 +515,13 @@ def bench_3d(args):
             quality_measure="minimum dihedral angle (degrees) of the raw loop mesh after the "
                             "timed iterations (cells flat to rounding count as 0), and the 1st "
                             "percentile of the cells' minimum angles",
-            host_tet_ms_per_iteration=round(stats["host_tet_us"] / 1e3 / args.steps, 2),
-            plain_host_tet_ms_per_iteration=round(plain_stats["host_tet_us"] / 1e3 /
-                                                  args.steps, 2),
+            tet_ms_per_iteration=dict(
+                device=round(stats["device_tet_us"] / 1e3 / args.steps, 2),
+                host=round(stats["host_tet_us"] / 1e3 / args.steps, 2)),
+            plain_tet_ms_per_iteration=dict(
+                device=round(plain_stats["device_tet_us"] / 1e3 / args.steps, 2),
+                host=round(plain_stats["host_tet_us"] / 1e3 / args.steps, 2)),
+            device_builds=stats["device_builds"], host_builds=stats["host_rebuilds"],
             device_ms_per_iteration=round(dev_ms, 3),
             parallel_builds=stats["parallel_builds"],
             retried_points_per_iteration=round(stats["retried_points"] / args.steps, 1),

@@ -345,17 +345,23 @@ int sm_mesher_get_edges(sm_mesher *m, int32_t *edges, int64_t cap);
  * the slot count or an error code.  For checking the device repair. */
 int64_t sm_mesher_get_triangulation(sm_mesher *m, int32_t *tri, int32_t *adj, int64_t cap);
 /* Statistics since creation: [0] iterations, [1] flip rounds, [2] flips,
- * [3] rebuilds (on the host in 2D; every 3D triangulation is one), [4] exact predicate
+ * [3] triangulations built on the host (2D and 3D), [4] exact predicate
  * evaluations, [5] speculative (graph) iterations redone because their flips
  * had not converged, [6] kinetic repairs (points moved in sub-steps from the
  * last valid triangulation), [7] predicates the device's exact stage could
  * not settle (each forces a host rebuild), [8] vertices taken out and put
- * back on the host to untangle what flips could not, [9] 3D builds on the
- * device or on several host threads, [10] points the threads left to the final single-thread
- * pass (their cells were locked by another thread twice), [11] finite
- * tetrahedra of the last 3D build (0 in 2D), [12]
- * microseconds spent in the 3D tetrahedralisation (wall clock; on the host
- * with copies and overlapped filters). */
+ * back on the host to untangle what flips could not, [9] 3D builds on
+ * several host threads, [10] points the threads left to the final
+ * single-thread pass (their cells were locked by another thread twice),
+ * [11] finite tetrahedra of the last 3D build (0 in 2D), [12] microseconds
+ * spent in 3D builds on the host (wall clock, copies and overlapped filters
+ * included), [13] 3D builds on the device, [14] microseconds spent in them
+ * (wall clock), [15] why the device left the last point set it looked at to
+ * the host: 0 it did not, 1 too few or too many points, points in one plane,
+ * or coordinates out of range, 2 a predicate its exact stage could not
+ * settle, 3 or 4 no room for the stars' or the output's cells, 5 too many
+ * stars that need exact predicates, 7 too many or too tangled large stars, 8
+ * no memory for its scratch. */
 int sm_mesher_stats(sm_mesher *m, int64_t *stats, int nstats);
 /* 3D handles: what the device build leaves to the host (small or degenerate
  * point sets) is tetrahedralised on nthreads host threads inserting the points of nslabs slabs along `axis` into one shared

@@ -10,7 +10,7 @@
 #include "sizing_eval.h"
 #include "stars3d.h"
 
-constexpr int kNumStats = 13;
+constexpr int kNumStats = 16;
 
 constexpr double kFarSquare = 100.0;
 

@@ -182,13 +182,13 @@ int device_rebuild3d(sm_mesher *m, bool *done) {
   int64_t count = 0;
   int rc = device_delaunay3d(&m->stars, m->d_p, m->N, m->prm.h0, m->d_tri, m->capT, &count, done,
                              m->stream);
+  m->stats[15] = m->stars.left;
   if (rc || !*done) return rc;
   m->T = count;
-  m->stats[3] += 1;
-  m->stats[9] += 1;
   m->stats[11] = count;
+  m->stats[13] += 1;
   m->have_tri = true;
-  m->stats[12] += (int64_t)std::chrono::duration_cast<std::chrono::microseconds>(
+  m->stats[14] += (int64_t)std::chrono::duration_cast<std::chrono::microseconds>(
                       std::chrono::steady_clock::now() - t0)
                       .count();
   return SM_OK;

@@ -9,6 +9,19 @@
 
 namespace smk {
 
+// Why a build is left to the host (the kernels' status word uses the first
+// five).
+enum StarLeft {
+  kLeftNot = 0,
+  kLeftInput = 1,       // too few or many points, a flat set, coordinates out of range
+  kLeftUnresolved = 2,  // a predicate beyond the exact stage
+  kLeftPool = 3,        // more link triangles than the pool holds
+  kLeftCells = 4,       // more cells than the output holds
+  kLeftUncertain = 5,   // too many stars in need of exact predicates
+  kLeftHubs = 7,        // too many large stars, or theirs could not be settled
+  kLeftMemory = 8       // no memory for the scratch
+};
+
 // Scratch of the device build (one per handle, grown to its largest point
 // set: about 0.6 kB a point).
 struct StarScratch {
@@ -17,7 +30,7 @@ struct StarScratch {
   size_t max_bytes = SIZE_MAX;  // builds that need more go to the host
   int32_t *h_status = nullptr;  // pinned
   int skip = 0;                 // builds left to the host after a failed one
-  int64_t builds = 0, hubs = 0;
+  int left = kLeftNot;          // why the last build it looked at was left
 };
 
 void stars_free(StarScratch *s);

@@ -123,7 +123,7 @@ __global__ void k_star_bbox(int64_t n, const double *p, uint64_t *bb, int32_t *s
       lo[k] = fmin(lo[k], __shfl_xor(lo[k], off));
       hi[k] = fmax(hi[k], __shfl_xor(hi[k], off));
     }
-  if (__ballot(bad) && threadIdx.x % 64 == 0) status[kStFail] = 1;
+  if (__ballot(bad) && threadIdx.x % 64 == 0) status[kStFail] = kLeftInput;
   if (threadIdx.x % 64 == 0)
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -151,7 +151,7 @@ __global__ void k_star_grid(int64_t n, double spacing, int64_t cap_cells, int64_
   ok = ok && s > 0.0;
   if (!ok) {
     s = 1.0;
-    status[kStFail] = 1;
+    status[kStFail] = kLeftInput;
   }
   if (spacing > 0.0 && spacing < s) s = spacing;
   for (int it = 0; it < 4096; ++it) {
@@ -165,7 +165,7 @@ __global__ void k_star_grid(int64_t n, double spacing, int64_t cap_cells, int64_
     s *= 1.05;
   }
   // squared distances are compared in FP32
-  if (!(s > 1e-15 && s < 1e15)) status[kStFail] = 1;
+  if (!(s > 1e-15 && s < 1e15)) status[kStFail] = kLeftInput;
   g->s = s;
   g->inv = 1.0 / s;
   // rounding of a cell's corner, and of the cell a point falls into
@@ -175,14 +175,14 @@ __global__ void k_star_grid(int64_t n, double spacing, int64_t cap_cells, int64_
     d[k] = ok ? (int64_t)floor(ext[k] / s) + 1 : 1;
     if (d[k] > 1024) {
       d[k] = 1;
-      status[kStFail] = 1;
+      status[kStFail] = kLeftInput;
     }
     g->g[k] = (int32_t)d[k];
     c *= d[k];
   }
   if (c > cap_cells) {
     for (int k = 0; k < 3; ++k) g->g[k] = (int32_t)(d[k] = 1);
-    status[kStFail] = 1;
+    status[kStFail] = kLeftInput;
   }
   int l = 0;
   int64_t off = 0;
@@ -197,7 +197,7 @@ __global__ void k_star_grid(int64_t n, double spacing, int64_t cap_cells, int64_
     // no room (a grid one or two cells wide): nothing may be written
     for (int k = 0; k < 3; ++k) g->g[k] = g->dim[0][k] = 1;
     g->nlev = 1;
-    status[kStFail] = 1;
+    status[kStFail] = kLeftInput;
   }
 }
 
@@ -1091,13 +1091,13 @@ __global__ __launch_bounds__(64 * kStarWaves, EXACT ? 1 : (FAR ? 3 : 4)) void k_
   if (status[kStFail]) return;
   // too many uncertain stars after the near pass: the rest is no use
   if (FAR && status[kStX] > most_exact) {
-    if (threadIdx.x == 0) status[kStFail] = 5;
+    if (threadIdx.x == 0) status[kStFail] = kLeftUncertain;
     return;
   }
   const int lane = threadIdx.x % 64;
   const int64_t items = list ? (int64_t)*nlist : n;
   if (list && items > most) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) status[kStFail] = 5;
+    if (blockIdx.x == 0 && threadIdx.x == 0) status[kStFail] = kLeftUncertain;
     return;
   }
   const int64_t nw = (int64_t)gridDim.x * kStarWaves;
@@ -1127,7 +1127,7 @@ __global__ __launch_bounds__(64 * kStarWaves, EXACT ? 1 : (FAR ? 3 : 4)) void k_
         if (rc == kFar) far[atomicAdd(&status[kStF], 1)] = self;
         else if (rc == kUncertain) exact[atomicAdd(&status[kStX], 1)] = self;
         else if (rc == kOverflow) hubs[atomicAdd(&status[kStHub], 1)] = id;
-        else status[kStFail] = 2;
+        else status[kStFail] = kLeftUnresolved;
       }
       wave_sync();
       continue;
@@ -1148,7 +1148,7 @@ __global__ __launch_bounds__(64 * kStarWaves, EXACT ? 1 : (FAR ? 3 : 4)) void k_
     if (lane == 0) off = atomicAdd(&status[kStPool], total);
     off = uni(off);
     if ((int64_t)off + total > pool_cap || off < 0) {
-      if (lane == 0) status[kStFail] = 3;
+      if (lane == 0) status[kStFail] = kLeftPool;
       return;
     }
     if (lane == 0) {
@@ -1255,7 +1255,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_star_rows(
   wave_sync();
   const int64_t row = rowptr[v];
   if (row + r > cap) {
-    if (lane == 0) status[kStFail] = 4;
+    if (lane == 0) status[kStFail] = kLeftCells;
     return;
   }
   for (int p = lane; p < r; p += 64) {
@@ -1334,7 +1334,10 @@ void stars_free(StarScratch *s) {
 int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacing, int32_t *tet,
                       int64_t cap, int64_t *count, bool *done, hipStream_t s) {
   *done = false;
-  if (n < kStarMinPoints || n > (int64_t)1 << 25) return SM_OK;
+  if (n < kStarMinPoints || n > (int64_t)1 << 25) {
+    sc->left = kLeftInput;
+    return SM_OK;
+  }
   if (sc->skip > 0) {
     --sc->skip;
     return SM_OK;
@@ -1363,6 +1366,7 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
   // on the device
   const auto no_room = [&]() {
     (void)hipGetLastError();
+    sc->left = kLeftMemory;
     sc->skip = 3;
     return SM_OK;
   };
@@ -1450,14 +1454,16 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
   };
   if ((rc = place())) return rc;
   const int32_t *hs = sc->h_status;
-  const auto leave = [&]() {
+  const auto leave = [&](int why = kLeftHubs) {
+    sc->left = sc->h_status[kStFail] ? sc->h_status[kStFail] : why;
     // what fails now (a degenerate lattice) likely fails again; but a large
     // one is known for it early (5 of 130 ms) and loses a share of its
     // uncertain stars with every move
-    sc->skip = sc->h_status[kStFail] == 5 && n >= 65536 ? 2 : 3;
+    sc->skip = sc->left == kLeftUncertain && n >= 65536 ? 2 : 3;
     return SM_OK;
   };
-  if (hs[kStFail] || hs[kStHub] > kMaxHubs || hs[kStTotal] < 0) return leave();
+  if (hs[kStFail] || hs[kStHub] > kMaxHubs) return leave();
+  if (hs[kStTotal] > cap || hs[kStTotal] < 0) return leave(kLeftCells);
   // Hubs: their rows from their neighbours' stars and, for cells of four
   // hubs, from the hubs' own triangulation, each cell checked against every
   // point; some thousand cells, ordered on the host.  The host arrays outlive
@@ -1542,7 +1548,8 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
     SM_HIP(hipMemcpyAsync(tmp, rows.data(), nh * 4, hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(k_star_write, dim3(blocks_for(nh, B)), dim3(B), 0, s, nh, hub, tmp, row);
     if ((rc = place())) return rc;
-    if (hs[kStFail] || hs[kStTotal] > cap || hs[kStTotal] < 0) return leave();
+    // (the rows kernel does not see the hubs' rows)
+    if (hs[kStFail] || hs[kStTotal] > cap || hs[kStTotal] < 0) return leave(kLeftCells);
     hipLaunchKernelGGL(k_star_read, dim3(blocks_for(nh, B)), dim3(B), 0, s, nh, hub, rowp, tmp);
     SM_LAUNCH_CHECK();
     r0.resize((size_t)nh);
@@ -1564,14 +1571,12 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
       SM_LAUNCH_CHECK();
       SM_HIP(hipStreamSynchronize(s));
     }
-    sc->hubs += nh;
   } catch (const std::bad_alloc &) {
     SM_HIP(hipStreamSynchronize(s));
     return leave();
   }
-  if (hs[kStTotal] > cap) return leave();
   *count = hs[kStTotal];
-  sc->builds += 1;
+  sc->left = kLeftNot;
   *done = true;
   return SM_OK;
 }

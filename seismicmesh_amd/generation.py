@@ -358,7 +358,8 @@ class Mesher:
 
     STATS = ("iterations", "flip_rounds", "flips", "host_rebuilds", "exact_predicates",
              "rollbacks", "kinetic_repairs", "unresolved", "relocations", "parallel_builds",
-             "retried_points", "tets_last_build", "host_tet_us")
+             "retried_points", "tets_last_build", "host_tet_us", "device_builds", "device_tet_us",
+             "device_left")
 
     def stats(self):
         k = len(self.STATS)

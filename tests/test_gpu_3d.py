@@ -157,6 +157,8 @@ def test_slab_build_iterations_identical_to_serial(axis, nslabs, threads):
     st = generation.prepare(dom, h, verbose=0, precision=32)
     a = generation.make_mesher(st, slabs=1)
     b = generation.make_mesher(st, slabs=1)
+    for m in (a, b):
+        m.set_scratch_limit(1)  # every build on the host
     b.set_slabs(nslabs, axis=axis, threads=threads)
     a.set_points(st["p"])
     b.set_points(st["p"])
@@ -172,6 +174,7 @@ def test_slab_build_iterations_identical_to_serial(axis, nslabs, threads):
           "host %.1f ms per build" % (len(st["p"]), nslabs, axis, threads, s["parallel_builds"],
                                       s["retried_points"], s["host_tet_us"] / 1e3 /
                                       s["host_rebuilds"]))
-    assert s["parallel_builds"] == s["host_rebuilds"] >= 5
+    assert s["parallel_builds"] == s["host_rebuilds"] >= 5 and s["device_builds"] == 0
+    assert a.stats()["host_rebuilds"] >= 5 and a.stats()["parallel_builds"] == 0
     a.close()
     b.close()
