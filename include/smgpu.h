@@ -360,7 +360,8 @@ int64_t sm_mesher_get_triangulation(sm_mesher *m, int32_t *tri, int32_t *adj, in
  * the host: 0 it did not, 1 too few or too many points, points in one plane,
  * or coordinates out of range, 2 a predicate its exact stage could not
  * settle, 3 or 4 no room for the stars' or the output's cells, 5 too many
- * stars that need exact predicates, 7 too many or too tangled large stars, 8
+ * stars that need exact predicates, 6 a strongly clustered set, too many of
+ * its points in few cells of the search grid, 7 too many or too tangled large stars, 8
  * no memory for its scratch. */
 int sm_mesher_stats(sm_mesher *m, int64_t *stats, int nstats);
 /* 3D handles: what the device build leaves to the host (small or degenerate

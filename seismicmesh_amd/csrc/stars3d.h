@@ -18,6 +18,7 @@ enum StarLeft {
   kLeftPool = 3,        // more link triangles than the pool holds
   kLeftCells = 4,       // more cells than the output holds
   kLeftUncertain = 5,   // too many stars in need of exact predicates
+  kLeftCrowded = 6,     // too many points to a cell of the search grid
   kLeftHubs = 7,        // too many large stars, or theirs could not be settled
   kLeftMemory = 8       // no memory for the scratch
 };
@@ -47,8 +48,8 @@ constexpr int64_t kStarMinPoints = 512;
 // points (any positive value is correct; it sizes the search grid).
 // Synchronises the stream.  *done is false when the device leaves the build
 // to the host (too few points, points in one plane, predicates its exact
-// stage cannot settle, too many uncertain ones or very large stars, no memory
-// for the scratch); nothing is written then that the host build does not
+// stage cannot settle, too many uncertain ones, very large stars or points to
+// a cell of its grid, no memory for the scratch); nothing is written then that the host build does not
 // replace.
 int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacing, int32_t *tet,
                       int64_t cap, int64_t *count, bool *done, hipStream_t s);

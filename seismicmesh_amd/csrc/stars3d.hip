@@ -62,6 +62,17 @@ using smpred::kEps;
 constexpr int kMaxLevels = 6;
 constexpr int kCellsPerPoint = 6;
 constexpr int kMaxHubs = 8192;
+// Points of a cell beyond this many are crowded.  A star's first candidates
+// are any 64 of the cells around it, and where those hold many times more,
+// hardly one of the 64 is a neighbour: the link outgrows 64 triangles, so
+// that there are about as many hubs as crowded points (60 k points, a
+// twentieth of them 64, 256, 1024 to a cell: 1.6, 2.3, 2.5 k hubs of 1.9,
+// 2.7, 2.9 k crowded points).  The build is therefore left at once when
+// there are more of them than it may have hubs.  This also bounds what a cell
+// can hold, and with it the loops over a cell's points.  Half of 60 k points
+// some thousands to a cell: 83 ms before, 40 of them for near and far passes
+// that ended with 28 k hubs; the host's 30 now.
+constexpr int kCrowded = 24;
 constexpr int kPoolPerPoint = 32;  // link triangles per vertex (24.5 on average)
 
 struct SPt {  // a point in grid order
@@ -88,7 +99,16 @@ struct StarGrid {
 };
 
 // status words (device, then pinned host)
-enum { kStX = 0, kStF = 1, kStHub = 2, kStFail = 3, kStPool = 4, kStTotal = 5, kStWords = 8 };
+enum {
+  kStX = 0,
+  kStF = 1,
+  kStHub = 2,
+  kStFail = 3,
+  kStPool = 4,
+  kStTotal = 5,
+  kStCrowd = 6,
+  kStWords = 8
+};
 
 __device__ inline uint64_t enc(double x) {
   const uint64_t u = (uint64_t)__double_as_longlong(x);
@@ -210,7 +230,7 @@ __device__ inline int64_t cell_index(const StarGrid &g, int i, int j, int k) {
 }
 
 __global__ void k_star_count(int64_t n, const double *p, const StarGrid *gp, int32_t *cnt,
-                             int32_t *cell, const int32_t *status) {
+                             int32_t *cell, int32_t *status) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   if (status[kStFail]) {
@@ -221,15 +241,19 @@ __global__ void k_star_count(int64_t n, const double *p, const StarGrid *gp, int
   const int32_t c = (int32_t)cell_index(g, cell_coord(g, p[3 * i], 0), cell_coord(g, p[3 * i + 1], 1),
                                         cell_coord(g, p[3 * i + 2], 2));
   cell[i] = c;
-  atomicAdd(&cnt[c], 1);
+  const uint64_t m = __ballot(atomicAdd(&cnt[c], 1) >= kCrowded);
+  if (m && threadIdx.x % 64 == __builtin_ctzll(m))
+    atomicAdd(&status[kStCrowd], (int32_t)__builtin_popcountll(m));
 }
 
 // the counts are consumed from the top, so they are zero again afterwards
 __global__ void k_star_scatter(int64_t n, const double *p, const int32_t *cell,
-                               const int32_t *start, int32_t *cnt, SPt *ps,
-                               const int32_t *status) {
+                               const int32_t *start, int32_t *cnt, SPt *ps, int32_t most,
+                               int32_t *status) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || status[kStFail]) return;
+  const bool crowded = status[kStCrowd] > most;
+  if (crowded && i == 0) status[kStFail] = kLeftCrowded;
+  if (i >= n || crowded || status[kStFail]) return;
   const int32_t c = cell[i];
   SPt q;
   q.x = p[3 * i];
@@ -261,9 +285,9 @@ __global__ void k_star_dups(int64_t n, const StarGrid *gp, const int32_t *start,
 // search pass over them (with cell boxes every facet in such a side entered
 // every cell of the side).
 __global__ void k_star_nodes(const StarGrid *gp, int level, const int32_t *start, const SPt *ps,
-                             Node *nodes) {
+                             Node *nodes, const int32_t *status) {
   const StarGrid &g = *gp;
-  if (level >= g.nlev) return;
+  if (level >= g.nlev || status[kStFail]) return;
   const int lane = threadIdx.x % 64;
   const int32_t *d = g.dim[level];
   const int64_t count = (int64_t)d[0] * d[1] * d[2];
@@ -1407,6 +1431,10 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
 
   const int B = 256;
   const unsigned gn = blocks_for(n, B);
+  // the hubs are settled on one host thread, which has the whole set done in
+  // eight times what an eighth of it takes (8 k points with 1.3 k hubs: 25 ms
+  // against the host's 18, and 4.2 with 174)
+  const int32_t most_hubs = (int32_t)std::min<int64_t>(kMaxHubs, n / 8);
   int rc;
   hipLaunchKernelGGL(k_star_init, dim3(1), dim3(64), 0, s, bb, st);
   hipLaunchKernelGGL(k_star_bbox, dim3(std::min(gn, 256u)), dim3(B), 0, s, n, p, bb, st);
@@ -1414,12 +1442,13 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
   if ((rc = fill<int32_t>(cnt, cells + 1, 0, s))) return rc;
   hipLaunchKernelGGL(k_star_count, dim3(gn), dim3(B), 0, s, n, p, g, cnt, cell, st);
   if ((rc = scan_exclusive(cnt, start, cells + 1, nullptr, ws, s))) return rc;
-  hipLaunchKernelGGL(k_star_scatter, dim3(gn), dim3(B), 0, s, n, p, cell, start, cnt, ps, st);
+  hipLaunchKernelGGL(k_star_scatter, dim3(gn), dim3(B), 0, s, n, p, cell, start, cnt, ps, most_hubs,
+                     st);
   hipLaunchKernelGGL(k_star_dups, dim3(gn), dim3(B), 0, s, n, g, start, ps, st);
   for (int l = 0; l < kMaxLevels; ++l) {
     const int64_t most = std::max<int64_t>(1, cells >> (5 * l));
     hipLaunchKernelGGL(k_star_nodes, dim3((unsigned)std::min<int64_t>(2048, blocks_for(most, 4))),
-                       dim3(B), 0, s, g, l, start, ps, nodes);
+                       dim3(B), 0, s, g, l, start, ps, nodes, st);
   }
   // uncertain predicates beyond this many vertices: a degenerate lattice,
   // which the host settles sooner.  An exact star takes 0.25 us when the
@@ -1462,7 +1491,7 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
     sc->skip = sc->left == kLeftUncertain && n >= 65536 ? 2 : 3;
     return SM_OK;
   };
-  if (hs[kStFail] || hs[kStHub] > kMaxHubs) return leave();
+  if (hs[kStFail] || hs[kStHub] > most_hubs) return leave();
   if (hs[kStTotal] > cap || hs[kStTotal] < 0) return leave(kLeftCells);
   // Hubs: their rows from their neighbours' stars and, for cells of four
   // hubs, from the hubs' own triangulation, each cell checked against every

@@ -158,3 +158,28 @@ def test_a_build_without_room_for_its_scratch_goes_to_the_host():
         s = m.stats()
         assert s["device_builds"] == built and s["device_left"] == (8 if limit == 100000 else 0)
     m.close()
+
+
+@pytest.mark.parametrize("share,radius,left", [(0.5, 0.02, 6), (0.5, 1e-4, 6), (0.5, 1e-9, 6),
+                                               (0.05, 0.02, 0), (0.05, 1e-9, 2)])
+def test_crowded_cells_are_left_to_the_host(share, radius, left):
+    # `share` of 8000 points in a small ball, amid the rest: most of them
+    # beyond the 24th of their cell of the search grid when the ball has few
+    # cells; up to an eighth of all points may be (the last set's reason is
+    # another: coordinates of 1e-9 next to ones of 1 span more bits than the
+    # exact stage holds)
+    rng = np.random.default_rng(3)
+    k = int(8000 * share)
+    d = rng.normal(size=(k, 3))
+    d *= radius * rng.random((k, 1)) ** (1 / 3) / np.linalg.norm(d, axis=1)[:, None]
+    p = np.vstack([d, rng.uniform(-1, 1, (8000 - k, 3))])
+    from seismicmesh_amd import generation, geometry as geo
+    m = generation.Mesher([geo.Ball([0.0, 0.0, 0.0], 1e7)],
+                          generation._Sizing("const", value=0.1), 0.1, 0.2, 0.01, 1e-9, 0,
+                          precision=32, dim=3)
+    m.set_points(p)
+    m.triangulate()
+    assert np.array_equal(m.cells(), _host(np.ascontiguousarray(p)))
+    s = m.stats()
+    assert s["device_left"] == left and s["device_builds"] == (left == 0)
+    m.close()
