@@ -561,6 +561,7 @@ extern "C" int sm_mesher_set_points(sm_mesher *m, const double *p, int64_t n) {
              (long long)m->h_voff[m->ndom], (long long)n);
   m->N = n;
   m->NA = n + m->nfar;
+  m->stars.skip = 0;  // what failed on other points says nothing about these
   SM_HIP(hipMemcpyAsync(m->d_p, p, n * m->dim * sizeof(double), hipMemcpyHostToDevice,
                         m->stream));
   m->have_tri = false;

@@ -183,3 +183,19 @@ def test_crowded_cells_are_left_to_the_host(share, radius, left):
     s = m.stats()
     assert s["device_left"] == left and s["device_builds"] == (left == 0)
     m.close()
+
+
+def test_new_points_are_tried_on_the_device_whatever_failed_before():
+    from seismicmesh_amd import generation, geometry as geo
+    m = generation.Mesher([geo.Ball([0.0, 0.0, 0.0], 1e7)],
+                          generation._Sizing("const", value=0.1), 0.1, 0.2, 0.01, 1e-9, 0,
+                          precision=32, dim=3)
+    g = np.arange(13) / 16.0
+    lattice = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+    good = np.random.default_rng(1).uniform(-1, 1, (2000, 3))
+    for p, built in ((lattice, 0), (good, 1), (good, 2), (lattice, 2), (good, 3)):
+        m.set_points(p)
+        m.triangulate()
+        assert m.stats()["device_builds"] == built
+        assert np.array_equal(m.cells(), _host(np.ascontiguousarray(p)))
+    m.close()
