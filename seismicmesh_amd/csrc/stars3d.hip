@@ -431,7 +431,7 @@ struct Tri {
   float diam;   // upper bound of the sphere's diameter (inf: none)
 };
 
-enum { kOk = 0, kUncertain = 1, kOverflow = 2, kUnresolved = 3, kFar = 4, kConflict = 5 };
+enum { kOk = 0, kUncertain = 1, kOverflow = 2, kUnresolved = 3, kFar = 4, kVoid = 5 };
 
 // FAR: with the tree search.  EXACT: uncertain tests settled by the integer
 // stage (else they end the star with kUncertain).
@@ -443,6 +443,7 @@ struct Star {
   const SPt *ps;
   const int32_t *start;
   const Node *nodes;
+  const int32_t *fail;  // EXACT: set once the whole build is void
   double vx, vy, vz;
   int self;
   Tri t;
@@ -451,8 +452,17 @@ struct Star {
   float need2 = INFINITY;  // square of the largest diameter
 
   __device__ Star(StarLds &s, FarLds *f, const StarGrid &gg, const SPt *p, const int32_t *st,
-                  const Node *m)
-      : sh(s), fsh(f), g(gg), ps(p), start(st), nodes(m) {}
+                  const Node *m, const int32_t *fl)
+      : sh(s), fsh(f), g(gg), ps(p), start(st), nodes(m), fail(fl) {}
+
+  // A star of a lattice takes milliseconds of exact predicates, one after
+  // the other: after each of them it looks whether another star has met one
+  // that cannot be settled.  (One read a predicate of tens of microseconds.
+  // With all stars in flight finished first, the exact pass of such an
+  // attempt took 4-5 ms on 138 k points; 2-3 now.)
+  __device__ bool voided() const {
+    return uni(__hip_atomic_load(fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0;
+  }
 
   __device__ P3 tab(int i) const { return P3{{sh.tx[i], sh.ty[i], sh.tz[i]}}; }
   __device__ P3 vert() const { return P3{{vx, vy, vz}}; }
@@ -525,11 +535,27 @@ struct Star {
     need2 = m * m * 1.00001f;
   }
 
-  // v, a, b (of a hull facet) and q share a coordinate: exactly coplanar
+  // v, a, b (of a hull facet) and q are exactly coplanar: they share a
+  // coordinate, or three of them, q included, share two (a row along an
+  // axis).  On the edges of a box this settles what the exact stage cannot:
+  // rows with a coordinate 0 next to neighbours at 1e-13.  (138 k points of a
+  // graded box, 8 iterations from their lattice: 403 ms without the rows, 2
+  // of the last 5 builds tried on the device in vain; 327 with them, all 5
+  // made there; 375 with every build on 16 host threads.)
   __device__ bool same_plane(int a, int b, double x, double y, double z) const {
-    return (vx == x && sh.tx[a] == x && sh.tx[b] == x) ||
-           (vy == y && sh.ty[a] == y && sh.ty[b] == y) ||
-           (vz == z && sh.tz[a] == z && sh.tz[b] == z);
+    const bool vq[3] = {vx == x, vy == y, vz == z};
+    const bool aq[3] = {sh.tx[a] == x, sh.ty[a] == y, sh.tz[a] == z};
+    const bool bq[3] = {sh.tx[b] == x, sh.ty[b] == y, sh.tz[b] == z};
+    int va = 0, vb = 0, ab = 0;
+    bool all = false;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      all = all || (vq[k] && aq[k] && bq[k]);
+      va += vq[k] && aq[k];
+      vb += vq[k] && bq[k];
+      ab += aq[k] && bq[k];
+    }
+    return all || va > 1 || vb > 1 || ab > 1;
   }
 
   // lane of the finite triangle across the edge (a, b) of a hull facet
@@ -572,6 +598,7 @@ struct Star {
       conf = o > 0 && !bad;
     }
     if (EXACT && __ballot(bad)) return kUnresolved;
+    if (EXACT && voided()) return kVoid;
     // a point in a hull facet's plane: as the finite tetrahedron behind it
     uint64_t m = __ballot(flat);
     while (m) {
@@ -962,8 +989,9 @@ struct Star {
             bad = bad || o == SM_PRED_UNRESOLVED;
             in = in || (o > 0 && o != SM_PRED_UNRESOLVED);
           }
+          if (EXACT && __ballot(bad)) return kUnresolved;
+          if (EXACT && voided()) return kVoid;
         }
-        if (EXACT && __ballot(bad)) return kUnresolved;
         if (__ballot(in) == 0) continue;
         float best = in ? (float)l : INFINITY;
 #pragma unroll
@@ -1138,7 +1166,7 @@ __global__ __launch_bounds__(64 * kStarWaves, EXACT ? 1 : (FAR ? 3 : 4)) void k_
       if (lane == 0) pcnt[id] = rowcnt[id] = poff[id] = 0;
       continue;
     }
-    Star<FAR, EXACT> st(shm[wv], &fshm[FAR ? wv : 0], *gp, ps, start, nodes);
+    Star<FAR, EXACT> st(shm[wv], &fshm[FAR ? wv : 0], *gp, ps, start, nodes, status + kStFail);
     st.vx = q.x;
     st.vy = q.y;
     st.vz = q.z;
@@ -1151,7 +1179,9 @@ __global__ __launch_bounds__(64 * kStarWaves, EXACT ? 1 : (FAR ? 3 : 4)) void k_
         if (rc == kFar) far[atomicAdd(&status[kStF], 1)] = self;
         else if (rc == kUncertain) exact[atomicAdd(&status[kStX], 1)] = self;
         else if (rc == kOverflow) hubs[atomicAdd(&status[kStHub], 1)] = id;
-        else status[kStFail] = kLeftUnresolved;
+        else if (rc == kUnresolved)
+          __hip_atomic_store(&status[kStFail], kLeftUnresolved, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
       }
       wave_sync();
       continue;
@@ -1195,13 +1225,13 @@ __global__ __launch_bounds__(64 * kStarWaves, EXACT ? 1 : (FAR ? 3 : 4)) void k_
 // grid order of each point id.
 __global__ __launch_bounds__(64 * kStarWaves) void k_star_check(
     const StarGrid *gp, const SPt *ps, const int32_t *start, const Node *nodes,
-    const int32_t *cells, int nc, const int32_t *pos, int32_t *bad) {
+    const int32_t *cells, int nc, const int32_t *pos, int32_t *bad, const int32_t *status) {
   __shared__ StarLds shm[kStarWaves];
   __shared__ FarLds fshm[kStarWaves];
   const int wv = uni(threadIdx.x / 64), lane = threadIdx.x % 64;
   const int c = blockIdx.x * kStarWaves + wv;
   if (c >= nc) return;
-  Star<true, true> st(shm[wv], &fshm[wv], *gp, ps, start, nodes);
+  Star<true, true> st(shm[wv], &fshm[wv], *gp, ps, start, nodes, status + kStFail);
   const int self = uni(pos[cells[4 * c]]);
   st.vx = ps[self].x;
   st.vy = ps[self].y;
@@ -1547,7 +1577,7 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
       SM_HIP(hipMemcpyAsync(dc, own.data(), own.size() * 4, hipMemcpyHostToDevice, s));
       hipLaunchKernelGGL(k_star_positions, dim3(gn), dim3(B), 0, s, n, ps, posn);
       hipLaunchKernelGGL(k_star_check, dim3(blocks_for(no, W)), dim3(64 * W), 0, s, g, ps, start,
-                         nodes, dc, no, posn, bad);
+                         nodes, dc, no, posn, bad, st);
       SM_LAUNCH_CHECK();
       hb.resize((size_t)no);
       SM_HIP(hipMemcpyAsync(hb.data(), bad, no * 4, hipMemcpyDeviceToHost, s));

@@ -67,6 +67,20 @@ def _points(kind):
         return _box(rng, 13, 0.0), 1 / 12
     if kind == "box_noise":
         return _box(rng, 13, 1e-15), 1 / 12
+    if kind.startswith("box_rows"):
+        # rows of points exactly on the edges of the box, noise on its sides:
+        # three of a row and a neighbour are coplanar, which the coordinates'
+        # span keeps from the exact stage.  Evenly spaced, the rows' points
+        # also lie on common spheres, which it cannot settle
+        g = np.linspace(0.0, 1.0, 13)
+        p = _box(rng, 13, 1e-14)
+        q = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+        side = (q == 0.0) | (q == 1.0)
+        edge = side.sum(1) >= 2
+        p[edge] = q[edge]
+        if kind == "box_rows":
+            p += np.where(side | ~edge[:, None], 0.0, rng.uniform(-0.2, 0.2, p.shape) / 13)
+        return p, 1 / 12
     if kind == "duplicates":
         p = rng.uniform(-1, 1, (1500, 3))
         return np.vstack([p, p[::7], p[::11]]), 0.15
@@ -91,15 +105,15 @@ def _points(kind):
 
 @pytest.mark.parametrize("kind", [
     "random511", "random512", "random513", "random2000", "random30000", "spacing_too_large",
-    "spacing_too_small", "clustered", "box_exact", "box_noise", "duplicates", "hub", "long",
-    "far_from_origin", "tiny", "lattice", "plane"])
+    "spacing_too_small", "clustered", "box_exact", "box_noise", "box_rows", "box_rows_even", "duplicates",
+    "hub", "long", "far_from_origin", "tiny", "lattice", "plane"])
 def test_cells_equal_the_host_build(kind):
     p, h = _points(kind)
     p = np.ascontiguousarray(p)
     ref = _host(p)
     got, on_device = _device(p, h)
     assert np.array_equal(got, ref)
-    if kind.startswith("random") or kind in ("box_exact", "box_noise", "hub", "long",
+    if kind.startswith("random") or kind in ("box_exact", "box_noise", "box_rows", "hub", "long",
                                              "duplicates"):
         assert on_device == (len(p) >= 512)
     if kind == "plane":
@@ -182,6 +196,37 @@ def test_crowded_cells_are_left_to_the_host(share, radius, left):
     assert np.array_equal(m.cells(), _host(np.ascontiguousarray(p)))
     s = m.stats()
     assert s["device_left"] == left and s["device_builds"] == (left == 0)
+    m.close()
+
+
+def _mixed_lattice(side, shift):
+    # A staggered lattice around the origin whose coordinates are rounded
+    # multiples of 0.1 (no common power of two), shifted by `shift`: zeros
+    # become coordinates of 1e-30 next to ones of 1, beyond the exact stage
+    g = (np.arange(side) - side // 2) * 0.1
+    p = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+    p[:, 0] += 0.05 * (np.arange(len(p)) // side % 2)
+    return p + shift
+
+
+@pytest.mark.parametrize("side", [16, 41])
+def test_a_predicate_beyond_the_exact_stage(side):
+    # 41^3 > 65536 points; enough of them moved that the build gets as far as
+    # its exact stars
+    p = _mixed_lattice(side, 1e-30)
+    rng = np.random.default_rng(side)
+    moved = rng.random(len(p)) < 0.7
+    p[moved] += rng.uniform(-0.01, 0.01, (int(moved.sum()), 3))
+    p = np.ascontiguousarray(p)
+    from seismicmesh_amd import generation, geometry as geo
+    m = generation.Mesher([geo.Ball([0.0, 0.0, 0.0], 1e7)],
+                          generation._Sizing("const", value=0.1), 0.1, 0.2, 0.01, 1e-9, 0,
+                          precision=32, dim=3)
+    m.set_points(p)
+    m.triangulate()
+    s = m.stats()
+    assert s["device_left"] == 2 and s["device_builds"] == 0
+    assert np.array_equal(m.cells(), _host(p))
     m.close()
 
 
