@@ -180,8 +180,8 @@ int host_sizing_pass(sm_mesher *m) {
 int device_rebuild3d(sm_mesher *m, bool *done) {
   const auto t0 = std::chrono::steady_clock::now();
   int64_t count = 0;
-  int rc = device_delaunay3d(&m->stars, m->d_p, m->N, m->prm.h0, m->d_tri, m->capT, &count, done,
-                             m->stream);
+  int rc = device_delaunay3d(&m->stars, m->d_p, m->N, m->prm.h0, m->sl_threads, m->d_tri, m->capT,
+                             &count, done, m->stream);
   m->stats[15] = m->stars.left;
   if (rc || !*done) return rc;
   m->T = count;

@@ -45,13 +45,15 @@ constexpr int64_t kStarMinPoints = 512;
 // The finite Delaunay tetrahedra of the n points p (device, (n, 3) FP64) to
 // `tet` (device, room for cap cells): the same cells in the same order as
 // sm_host_delaunay3d.  `spacing` is a typical distance between neighbouring
-// points (any positive value is correct; it sizes the search grid).
+// points (any positive value is correct; it sizes the search grid);
+// host_threads is the number of threads the host build would take.
 // Synchronises the stream.  *done is false when the device leaves the build
 // to the host (too few points, points in one plane, predicates its exact
 // stage cannot settle, too many uncertain ones, very large stars or points to
 // a cell of its grid, no memory for the scratch); nothing is written then that the host build does not
 // replace.
-int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacing, int32_t *tet,
-                      int64_t cap, int64_t *count, bool *done, hipStream_t s);
+int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacing,
+                      int host_threads, int32_t *tet, int64_t cap, int64_t *count, bool *done,
+                      hipStream_t s);
 
 }  // namespace smk

@@ -1385,8 +1385,29 @@ void stars_free(StarScratch *s) {
   s->bytes = 0;
 }
 
-int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacing, int32_t *tet,
-                      int64_t cap, int64_t *count, bool *done, hipStream_t s) {
+// The most vertices whose stars may need exact predicates: where the exact
+// pass takes as long as the host build would.  Measured with a share x of n
+// vertices (exact cubes in part of a box, jittered elsewhere): the pass takes
+// 1 + 35 x ms whatever n is up to 64 k, since the longest star decides (x =
+// 0.04 0.1 0.16 0.31 0.48: 1.9 2.9 4.5 8 15-18 ms); where moved vertices are
+// scattered among lattice ones, 1 + 9 x.  The other passes take 0.8 ms, the
+// host 2.2 us a point on one thread (4.3 on a whole lattice) and a quarter of
+// that or less on several.  Between the two slopes the lines meet at x =
+// (host - 1.8 ms) / 20 ms; a thirty-second costs at most 0.7 ms in any case,
+// and beyond a half whole lattices come, 20 ms and more for the longest star
+// and, on the 523 k points of the 76-primitive solid, 119 ms at x = 0.65 with
+// 16 host threads at 105-130.  Examples, device and host: 512 points, x =
+// 0.36, 7 ms and 1.3 (now left to the host); 3 k points from a ball's
+// lattice, x = 0.18, 2.7 and 7; 27 k, x = 0.41, 6.2 and 18 on 16 threads.
+int32_t most_exact_stars(int64_t n, int host_threads) {
+  const double host_ms = 2.2e-3 * (double)n / (host_threads > 1 ? 4.0 : 1.0);
+  const double share = std::min(0.5, std::max(1.0 / 32.0, (host_ms - 1.8) / 20.0));
+  return (int32_t)(share * (double)n);
+}
+
+int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacing,
+                      int host_threads, int32_t *tet, int64_t cap, int64_t *count, bool *done,
+                      hipStream_t s) {
   *done = false;
   if (n < kStarMinPoints || n > (int64_t)1 << 25) {
     sc->left = kLeftInput;
@@ -1480,16 +1501,7 @@ int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacin
     hipLaunchKernelGGL(k_star_nodes, dim3((unsigned)std::min<int64_t>(2048, blocks_for(most, 4))),
                        dim3(B), 0, s, g, l, start, ps, nodes, st);
   }
-  // uncertain predicates beyond this many vertices: a degenerate lattice,
-  // which the host settles sooner.  An exact star takes 0.25 us when the
-  // chip is full of them: 523 k points of the 76-primitive solid, two to
-  // eleven moves after their lattice, take 103 ms with 282 k exact stars, 91
-  // with 222 k, 54 with 36 k, against 105-130 ms on 16 host threads whatever
-  // they hold (119 with 344 k: even).  Few stars do not fill the chip, and
-  // the longest chain decides: 3 k points 23 ms with 2.7 k exact stars, the
-  // host's one thread 9.
-  const int32_t most_exact =
-      (int32_t)(n >= 65536 ? n / 2 : std::max<int64_t>(1024, n / 32));
+  const int32_t most_exact = most_exact_stars(n, host_threads);
   constexpr int W = kStarWaves;
   hipLaunchKernelGGL((k_stars<false, false>), dim3(blocks_for(n, W)), dim3(64 * W), 0, s, n, g, ps,
                      start, nodes, (const int32_t *)nullptr, (const int32_t *)nullptr, 0, lf, lx,

@@ -139,12 +139,14 @@ def test_a_failed_build_is_followed_by_the_host_then_the_device_again():
     m.close()
 
 
-@pytest.mark.parametrize("side,share,by_device", [(40, 0.3, False), (41, 0.3, True),
-                                                  (41, 0.7, False)])
+@pytest.mark.parametrize("side,share,by_device", [
+    (8, 0.25, False), (8, 0.45, False), (10, 0.25, False), (13, 0.06, True), (13, 0.25, False),
+    (16, 0.2, True), (16, 0.6, False), (40, 0.3, True), (41, 0.3, True), (41, 0.7, False)])
 def test_lattice_share_left_to_the_host(side, share, by_device):
     # exact cubes in part of the box (their stars take the exact pass), a
-    # jittered lattice in the rest: from 65536 points on (41^3) the device
-    # settles up to half of the vertices exactly, below that 1 in 32.
+    # jittered lattice in the rest: the device settles as many vertices
+    # exactly as cost it what the host's one thread would take, a
+    # thirty-second to a half.
     # Coordinates in [1, 2): one binary exponent, the exact stage's range
     rng = np.random.default_rng(side)
     g = 1.0 + np.arange(side) / 64.0
