@@ -78,7 +78,8 @@ __device__ inline void fragment(const float *sh, int row, int g, int half, float
 __device__ inline float sigmoid(float z) { return 1.0f / (1.0f + __expf(-z)); }
 
 template <int EPI, bool AK, bool BK, int MT>
-__global__ __launch_bounds__(256, EPI == kEpiStore || EPI == kEpiPart ? 3 : 2) void k_gemm32(GemmArgs g, int64_t kchunk) {
+__global__ __launch_bounds__(256, EPI == kEpiStore || EPI == kEpiPart ? 3 : 2) void k_gemm32(
+    GemmArgs g, int64_t kchunk) {
   constexpr int T = 64 * MT;
   constexpr int kA = stage_words<T>(AK), kB = stage_words<T>(BK);
   __shared__ __align__(16) float As[2][kA];
@@ -86,7 +87,10 @@ __global__ __launch_bounds__(256, EPI == kEpiStore || EPI == kEpiPart ? 3 : 2) v
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int r = lane % 32, half = lane / 32;
   const int wm = (wave / 2) * 32 * MT, wn = (wave % 2) * 32 * MT;
-  const int64_t m0 = (int64_t)blockIdx.y * T, n0 = (int64_t)blockIdx.x * T;
+  // tiles of one row of tiles are neighbours (they share A's rows); both
+  // indices in grid.x, since grid.y ends at 65535
+  const unsigned tn = (unsigned)((g.N + T - 1) / T), tm = blockIdx.x / tn;
+  const int64_t m0 = (int64_t)tm * T, n0 = (int64_t)(blockIdx.x - tm * tn) * T;
   const int64_t kb = (int64_t)blockIdx.z * kchunk, ke = kb + kchunk < g.K ? kb + kchunk : g.K;
   floatx16 acc[MT][MT];
 #pragma unroll
@@ -190,9 +194,11 @@ __global__ __launch_bounds__(256, EPI == kEpiStore || EPI == kEpiPart ? 3 : 2) v
     }
     __syncthreads();
     for (int c = threadIdx.x; c < T; c += 256)
-      if (n0 + c < g.N) g.C2[(int64_t)blockIdx.y * g.N + n0 + c] = red[c] + red[T + c];
+      if (n0 + c < g.N) g.C2[(int64_t)tm * g.N + n0 + c] = red[c] + red[T + c];
   }
 }
+
+constexpr int64_t kMaxTiles = (int64_t)1 << 23;
 
 int64_t split_chunk(const GemmArgs &g) {
   const int64_t per = (g.K + g.nsplit - 1) / std::max(g.nsplit, 1);
@@ -203,7 +209,7 @@ template <int EPI, bool AK, bool BK>
 void launch(const GemmArgs &g, bool small, hipStream_t s) {
   const int64_t T = small ? 64 : 128;
   const int64_t chunk = EPI == kEpiPart ? split_chunk(g) : std::max<int64_t>(g.K, 1);
-  const dim3 grid((unsigned)((g.N + T - 1) / T), (unsigned)((g.M + T - 1) / T),
+  const dim3 grid((unsigned)(((g.N + T - 1) / T) * ((g.M + T - 1) / T)), 1u,
                   EPI == kEpiPart ? (unsigned)gemm32_splits(g) : 1u);
   if (small)
     hipLaunchKernelGGL((k_gemm32<EPI, AK, BK, 1>), grid, dim3(256), 0, s, g, chunk);
@@ -226,13 +232,15 @@ int gemm32_splits(const GemmArgs &g) {
   return (int)std::max<int64_t>(1, (g.K + c - 1) / c);
 }
 
-// 16-byte loads: the contiguous index in fours, strides and bases aligned
+// 16-byte loads: the contiguous index in fours, strides and bases aligned;
+// no more tiles than a grid's threads (2^32) have room for
 bool gemm32_takes(bool ak, bool bk, const GemmArgs &g) {
   const auto ok = [&](const float *p, int64_t ld, int64_t run) {
     return ((uintptr_t)p & 15) == 0 && ld % 4 == 0 && run % 4 == 0 && ld >= run;
   };
   return g.M > 0 && g.N > 0 && g.K > 0 && ok(g.A, g.lda, ak ? g.K : g.M) &&
-         ok(g.B, g.ldb, bk ? g.K : g.N) && g.M <= (int64_t)65535 * 64;
+         ok(g.B, g.ldb, bk ? g.K : g.N) &&
+         (g.M + 63) / 64 <= kMaxTiles / ((g.N + 63) / 64);
 }
 
 int gemm32(GemmEpi epi, bool ak, bool bk, const GemmArgs &g, bool small, hipStream_t s) {

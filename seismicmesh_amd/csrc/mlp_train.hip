@@ -28,6 +28,9 @@ namespace smk {
 namespace {
 
 constexpr int kW = kTrainWidth;
+// rows of a pass (samples and their shifted copies): what the products take,
+// 1 TB of workspace for three hidden layers
+constexpr int64_t kMaxRows = (int64_t)1 << 27;
 
 __device__ inline float sigmoid(float z) { return 1.0f / (1.0f + __expf(-z)); }
 
@@ -253,7 +256,8 @@ Plan make_plan(int64_t n, int dim, int hidden, bool eik) {
 using namespace smk;
 
 extern "C" size_t sm_mlp_loss_grad_workspace(int64_t n, int in_dim, int hidden, float eik_h) {
-  if (n <= 0 || (in_dim != 2 && in_dim != 3) || hidden < 0 || hidden > 16) return 0;
+  if (n <= 0 || n > kMaxRows / 7 || (in_dim != 2 && in_dim != 3) || hidden < 0 || hidden > 16)
+    return 0;
   return (size_t)make_plan(n, in_dim, hidden, eik_h > 0.0f).total * sizeof(float);
 }
 
@@ -262,8 +266,9 @@ extern "C" int sm_mlp_loss_grad(int64_t n, int in_dim, int hidden, const double 
                                 float eik_h, float lam, float trunc, const float *params,
                                 float *grad, float *part, void *ws, size_t ws_bytes,
                                 void *stream) {
-  SM_CHECK(n > 0 && (in_dim == 2 || in_dim == 3) && hidden >= 0 && hidden <= 16, SM_ERR_ARG,
-           "mlp_loss_grad: bad size");
+  SM_CHECK(n > 0 && n <= kMaxRows / 7 && (in_dim == 2 || in_dim == 3) && hidden >= 0 &&
+               hidden <= 16,
+           SM_ERR_ARG, "mlp_loss_grad: bad size");
   SM_CHECK(x && t && shift && scale && params && grad && part && ws, SM_ERR_ARG,
            "mlp_loss_grad: null pointer");
   SM_CHECK(eik_h >= 0.0f && (lam == 0.0f || eik_h > 0.0f) && trunc >= 0.0f, SM_ERR_ARG,

@@ -25,7 +25,7 @@ def _p(t):
     (128, 128, 16, True, False, 1, 0), (132, 124, 36, True, True, 1, 0),
     (256, 256, 4, False, True, 1, 0), (33, 256, 256, False, True, 1, 0),
     (256, 256, 5001, True, False, 7, 0), (256, 256, 17, True, False, 9, 0),
-    (16500, 256, 256, False, True, 1, 0), (16384, 260, 64, False, False, 3, 0),
+    (16500, 256, 256, False, True, 1, 0), (65535 * 64 + 33, 36, 4, False, True, 1, 0), (16384, 260, 64, False, False, 3, 0),
     (31, 256, 256, False, True, 1, 0), (256, 256, 30, False, True, 1, 0),
     (64, 64, 64, False, True, 1, 1)])
 def test_gemm_matches_float64(M, N, K, ta, tb, nsplit, off):
@@ -76,3 +76,30 @@ def test_training_pass_matches_float64(n, dim, hidden, lam):
         r = ref[o:o + k]
         # as test_training_gradient_matches_oracle
         assert np.abs(g[o:o + k] - r).max() <= 2e-3 * np.abs(r).max() + 1e-7, name
+
+
+def test_training_pass_over_more_rows_than_a_grid_dimension():
+    """More than 65535 tiles of 64 rows (26 GB of workspace): the gradient is
+    the mean of those of two parts."""
+    import torch
+    from seismicmesh_amd.neural import NeuralSDF
+    net = NeuralSDF(2, [-1.0, 1.0] * 2, hidden=1, seed=3)
+    n, cut = 65535 * 64 + 77, 2000000
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.rand(n, 2, generator=g, device="cuda", dtype=torch.float64) * 2.0 - 1.0
+    t = (x.norm(dim=1) - 0.5).to(torch.float32)
+    whole, loss = None, []
+    mean = 0.0
+    for lo, hi in ((0, n), (0, cut), (cut, n)):
+        part = net.loss_and_grad(x[lo:hi], t[lo:hi], eik=0.0)
+        loss.append(float(part.double().sum()) * (hi - lo) / n)
+        if whole is None:
+            whole = net.grad.double()
+        else:
+            mean = mean + net.grad.double() * ((hi - lo) / n)
+    net._bufs = {}
+    assert abs(loss[0] - loss[1] - loss[2]) <= 1e-4 * loss[0]
+    for name, (o, k) in net.layout.items():
+        d = (whole - mean)[o:o + k].abs().max()
+        # as the passes against the oracle
+        assert float(d) <= 2e-3 * float(mean[o:o + k].abs().max()), name
