@@ -155,7 +155,8 @@ int sm_mlp_eval_centroids(const sm_mlp *net, const int32_t *cells, int64_t ncell
  * with respect to the network's flat FP32 parameters (device): w_in
  * [width][in_dim], b_in [width], w_hid [hidden][width][width] (rows = output
  * features), b_hid [hidden][width], w_out [width], b_out [1]; width is 256,
- * hidden at most 16, n at most 2^27 / 7.  shift and scale are host arrays of in_dim values.
+ * hidden at most 1024 (sm_mlp_eval takes 16), n at most 2^27 / 7.  shift and
+ * scale are host arrays of in_dim values.
  * eik_h > 0: the central-difference eikonal term with step eik_h and weight
  * lam.  grad: as many values as params; part: ceil(n / 256) loss partials.
  * params and ws are 16-byte aligned; ws holds at least

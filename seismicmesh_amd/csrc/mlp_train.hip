@@ -31,6 +31,8 @@ constexpr int kW = kTrainWidth;
 // rows of a pass (samples and their shifted copies): what the products take,
 // 1 TB of workspace for three hidden layers
 constexpr int64_t kMaxRows = (int64_t)1 << 27;
+// hidden layers (inference takes fewer)
+constexpr int kMaxLayers = 1024;
 
 __device__ inline float sigmoid(float z) { return 1.0f / (1.0f + __expf(-z)); }
 
@@ -187,7 +189,8 @@ struct SumJob {
   int32_t parts, cols;
   int32_t block0;
 };
-constexpr int kMaxJobs = 2 * 16 + 5;
+// jobs of one launch (of arguments: 32 bytes each); three layers take 10
+constexpr int kMaxJobs = 36;
 struct SumJobs {
   SumJob j[kMaxJobs];
   int n;
@@ -256,7 +259,8 @@ Plan make_plan(int64_t n, int dim, int hidden, bool eik) {
 using namespace smk;
 
 extern "C" size_t sm_mlp_loss_grad_workspace(int64_t n, int in_dim, int hidden, float eik_h) {
-  if (n <= 0 || n > kMaxRows / 7 || (in_dim != 2 && in_dim != 3) || hidden < 0 || hidden > 16)
+  if (n <= 0 || n > kMaxRows / 7 || (in_dim != 2 && in_dim != 3) || hidden < 0 ||
+      hidden > kMaxLayers)
     return 0;
   return (size_t)make_plan(n, in_dim, hidden, eik_h > 0.0f).total * sizeof(float);
 }
@@ -267,7 +271,7 @@ extern "C" int sm_mlp_loss_grad(int64_t n, int in_dim, int hidden, const double 
                                 float *grad, float *part, void *ws, size_t ws_bytes,
                                 void *stream) {
   SM_CHECK(n > 0 && n <= kMaxRows / 7 && (in_dim == 2 || in_dim == 3) && hidden >= 0 &&
-               hidden <= 16,
+               hidden <= kMaxLayers,
            SM_ERR_ARG, "mlp_loss_grad: bad size");
   SM_CHECK(x && t && shift && scale && params && grad && part && ws, SM_ERR_ARG,
            "mlp_loss_grad: null pointer");
@@ -324,6 +328,10 @@ extern "C" int sm_mlp_loss_grad(int64_t n, int in_dim, int hidden, const double 
   SumJobs jobs;
   jobs.n = 0;
   int blocks = 0;
+  const auto flush = [&]() {
+    if (jobs.n) hipLaunchKernelGGL(k_sum_parts, dim3(blocks), dim3(1024), 0, s, jobs);
+    jobs.n = blocks = 0;
+  };
   const auto sum = [&](const float *pp, int parts, int cols, float *out) {
     jobs.j[jobs.n++] = SumJob{pp, out, parts, cols, blocks};
     blocks += (cols + 63) / 64;
@@ -369,12 +377,15 @@ extern "C" int sm_mlp_loss_grad(int64_t n, int in_dim, int hidden, const double 
     if ((rc = gemm32(kEpiSiluBack, true, false, h, p.small, s))) return rc;
     dbparts = p.colparts;
     std::swap(dz, dz2);
+    // a deep network: more sums than one launch takes (the partials of every
+    // layer have their own place)
+    if (jobs.n + 4 > kMaxJobs) flush();
   }
   sum(w + p.p_db, dbparts, kW, grad + o_bin);
   hipLaunchKernelGGL(k_train_input_back, dim3(p.nchunk), dim3(256), 0, s, in, rows, p.chunk, dz,
                      w + p.p_wi);
   sum(w + p.p_wi, p.nchunk, kW * in_dim, grad);
-  hipLaunchKernelGGL(k_sum_parts, dim3(blocks), dim3(1024), 0, s, jobs);
+  flush();
   SM_LAUNCH_CHECK();
   return SM_OK;
 }

@@ -53,10 +53,12 @@ def test_gemm_matches_float64(M, N, K, ta, tb, nsplit, off):
 
 
 # row counts around the tile sizes and the switch between them (16384 rows),
-# with and without the eikonal copies, no hidden layer at all
+# with and without the eikonal copies, no hidden layer at all, more layers
+# than one launch of sums takes (15, 32, ...)
 @pytest.mark.parametrize("n,dim,hidden,lam", [
     (1, 3, 1, 0.0), (63, 2, 2, 0.0), (65, 3, 3, 0.1), (300, 2, 0, 0.1), (2341, 3, 1, 0.1),
-    (16383, 2, 1, 0.0), (16385, 3, 2, 0.0)])
+    (16383, 2, 1, 0.0), (16385, 3, 2, 0.0), (40, 2, 15, 0.0), (40, 2, 16, 0.1), (40, 3, 17, 0.0),
+    (40, 2, 40, 0.0)])
 def test_training_pass_matches_float64(n, dim, hidden, lam):
     import torch
     from oracle import mlp as omlp
