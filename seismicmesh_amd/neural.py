@@ -200,14 +200,16 @@ class NeuralSDF:
         """Forward and backward pass over the samples xt ((n, dim) float64
         device tensor) with targets tt (float32, distances in the network's
         frame, i.e. d * s; truncated at +-trunc when trunc > 0, where the
-        eikonal term is dropped).  Fills self.grad; returns the loss
+        eikonal term is dropped, as it is everywhere unless eik > 0).  Fills self.grad; returns the loss
         partials (device)."""
         n = xt.shape[0]
-        step = float(eik_h) if eik > 0 else 0.0
+        # a step that is not above zero goes with no weight but 0
+        drop = eik == 0 or (not eik > 0 and eik_h > 0)
+        lam, step = (0.0, 0.0) if drop else (float(eik), max(float(eik_h), 0.0))
         ws, part = self._buffers(n, step)
         _lib.check(_lib.lib.sm_mlp_loss_grad(
             n, self.dim, self.hidden, _ptr(xt), _ptr(tt), self.shift.ctypes.data,
-            self.scale.ctypes.data, step, float(eik), float(trunc), _ptr(self.params),
+            self.scale.ctypes.data, step, lam, float(trunc), _ptr(self.params),
             _ptr(self.grad), _ptr(part), _ptr(ws), ws.numel(), self._stream()),
             "sm_mlp_loss_grad")
         return part

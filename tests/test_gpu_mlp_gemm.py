@@ -105,3 +105,19 @@ def test_training_pass_over_more_rows_than_a_grid_dimension():
         d = (whole - mean)[o:o + k].abs().max()
         # as the passes against the oracle
         assert float(d) <= 2e-3 * float(mean[o:o + k].abs().max()), name
+
+
+@pytest.mark.parametrize("eik,eik_h", [(-0.1, 5e-3), (float("nan"), 5e-3), (0.0, -1.0)])
+def test_an_eikonal_weight_not_above_zero_drops_the_term(eik, eik_h):
+    import torch
+    from seismicmesh_amd.neural import NeuralSDF
+    net = NeuralSDF(2, [-1.0, 1.0] * 2, hidden=1, seed=3)
+    x = torch.from_numpy(np.random.default_rng(0).uniform(-1, 1, (100, 2))).cuda()
+    t = (x.norm(dim=1) - 0.5).to(torch.float32)
+    part = net.loss_and_grad(x, t, eik=0.0).clone()
+    grad = net.grad.clone()
+    assert torch.equal(net.loss_and_grad(x, t, eik=eik, eik_h=eik_h), part)
+    assert torch.equal(net.grad, grad)
+    for bad in ((0.1, 0.0), (0.1, -1.0), (-0.1, 0.0), (float("nan"), 0.0)):
+        with pytest.raises(RuntimeError, match="eik_h > 0"):
+            net.loss_and_grad(x, t, eik=bad[0], eik_h=bad[1])
