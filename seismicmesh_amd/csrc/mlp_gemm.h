@@ -6,6 +6,12 @@ namespace smk {
 
 constexpr int kTrainWidth = 256;
 
+// The pass's activation, rounded as sm_mlp_bias_silu rounds it (one division
+// of z; a product with the sigmoid would round once more), and its derivative
+// as sm_mlp_silu_backward.
+__device__ inline float train_sigmoid(float z) { return 1.0f / (1.0f + __expf(-z)); }
+__device__ inline float train_silu(float z) { return z / (1.0f + __expf(-z)); }
+
 // What becomes of the product P = A B:
 //   kEpiStore     C = alpha P + beta C
 //   kEpiPart      C[split][m][n] = the product over the split's k range

@@ -75,8 +75,6 @@ __device__ inline void fragment(const float *sh, int row, int g, int half, float
   }
 }
 
-__device__ inline float sigmoid(float z) { return 1.0f / (1.0f + __expf(-z)); }
-
 template <int EPI, bool AK, bool BK, int MT>
 __global__ __launch_bounds__(256, EPI == kEpiStore || EPI == kEpiPart ? 3 : 2) void k_gemm32(
     GemmArgs g, int64_t kchunk) {
@@ -170,9 +168,9 @@ __global__ __launch_bounds__(256, EPI == kEpiStore || EPI == kEpiPart ? 3 : 2) v
           } else if (EPI == kEpiSilu) {
             const float z = v + bias;
             g.C[m * g.ldc + n] = z;
-            g.C2[m * g.ldc + n] = z * sigmoid(z);
+            g.C2[m * g.ldc + n] = train_silu(z);
           } else {
-            const float z = zv[e], s = sigmoid(z);
+            const float z = zv[e], s = train_sigmoid(z);
             const float d = v * s * (1.0f + z * (1.0f - s));
             g.C[m * g.ldc + n] = d;
             cs[b] += d;

@@ -34,8 +34,6 @@ constexpr int64_t kMaxRows = (int64_t)1 << 27;
 // hidden layers (inference takes fewer)
 constexpr int kMaxLayers = 1024;
 
-__device__ inline float sigmoid(float z) { return 1.0f / (1.0f + __expf(-z)); }
-
 // x' of network row b * n + i: sample i scaled to the box, shifted along one
 // axis for b > 0 (sm_mlp_make_inputs)
 struct Inputs {
@@ -80,7 +78,7 @@ __global__ __launch_bounds__(256) void k_train_input(Inputs in, int64_t rows, co
       s = fmaf(wv[j][1], q[1], s);
       s = fmaf(wv[j][2], q[2], s);
       z[j] = s + bv[j];
-      a[j] = z[j] * sigmoid(z[j]);
+      a[j] = train_silu(z[j]);
     }
     *reinterpret_cast<float4 *>(Z + r * kW + f) = make_float4(z[0], z[1], z[2], z[3]);
     *reinterpret_cast<float4 *>(A + r * kW + f) = make_float4(a[0], a[1], a[2], a[3]);
@@ -130,7 +128,7 @@ __global__ __launch_bounds__(256) void k_train_output_back(int64_t rows, int64_t
     float d[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float s = sigmoid(z[j]);
+      const float s = train_sigmoid(z[j]);
       d[j] = g * wo[j] * s * (1.0f + z[j] * (1.0f - s));
       sw[j] = fmaf(g, a[j], sw[j]);
       sb[j] += d[j];

@@ -121,3 +121,34 @@ def test_an_eikonal_weight_not_above_zero_drops_the_term(eik, eik_h):
     for bad in ((0.1, 0.0), (0.1, -1.0), (-0.1, 0.0), (float("nan"), 0.0)):
         with pytest.raises(RuntimeError, match="eik_h > 0"):
             net.loss_and_grad(x, t, eik=bad[0], eik_h=bad[1])
+
+
+@pytest.mark.parametrize("hidden", [0, 1])
+def test_activation_rounds_as_the_single_step(hidden):
+    """One sample with gy = 1 and w_out = 0: the gradient of w_out is the last
+    activation itself, bit for bit that of sm_mlp_bias_silu (the identity as
+    hidden layer: the first one's activation once more)."""
+    import torch
+    from seismicmesh_amd import _lib
+    from seismicmesh_amd.neural import NeuralSDF
+    net = NeuralSDF(2, [-1.0, 1.0] * 2, hidden=hidden)
+    x = torch.tensor([[1.0, 0.0]], dtype=torch.float64, device="cuda")
+    t = torch.tensor([-0.5], dtype=torch.float32, device="cuda")
+    rng = np.random.default_rng(7)
+    o = {k: v[0] for k, v in net.layout.items()}
+    for scale in (1e-3, 0.3, 3.0, 20.0, 100.0):
+        z = (scale * rng.standard_normal(256)).astype(np.float32)
+        flat = np.zeros(net.nparams, dtype=np.float32)
+        flat[o["w_in"]:o["w_in"] + 512:2] = z
+        if hidden:
+            flat[o["w_hid"]:o["w_hid"] + 65536] = np.eye(256, dtype=np.float32).ravel()
+        net.set_params(flat)
+        net.loss_and_grad(x, t, eik=0.0)
+        zero = torch.zeros(256, dtype=torch.float32, device="cuda")
+        want = torch.from_numpy(z).cuda()
+        for _ in range(hidden + 1):
+            a = torch.empty_like(want)
+            _lib.check(_lib.lib.sm_mlp_bias_silu(1, 256, _p(want), _p(zero), _p(a), None),
+                       "sm_mlp_bias_silu")
+            want = a
+        assert torch.equal(net.grad[o["w_out"]:o["w_out"] + 256], want)
