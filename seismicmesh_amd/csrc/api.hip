@@ -184,8 +184,7 @@ __global__ __launch_bounds__(256) void k_limgrad_columns(double *f, int len, int
   }
 }
 
-// Lines longer than LDS holds (or more planes than a grid has): one thread
-// a line.
+// Lines longer than LDS holds, and short rows: one thread a line.
 __global__ void k_limgrad_axis(double *f, int64_t lines, int64_t len, int64_t stride,
                                int64_t outer, double step) {
   const int64_t line = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -285,10 +284,18 @@ extern "C" int sm_limgrad(double *f, int nz, int nx, int ny, double elen, double
     const int len = dims[axis];
     const int64_t lines = (int64_t)nz * nx * ny / len, outer = stride * len;
     if (len >= 2) {
+      // One thread a line: lines longer than LDS holds, more planes than
+      // grid.y counts (columns only: rows have none), and short rows.  Of
+      // those a thread's cache lines serve all of its few steps, and a
+      // workgroup of the rows kernel has little to sweep: 1000 lines of 20
+      // values 34 against 56 us for all three axes of the grid, 60000 of 16
+      // 57 against 69, 457 k of 8 172 against 224; but 457 k of 12 279
+      // against 258 and 457 k of 210 8.9 against 4.1 ms.
+      const bool few = stride == 1 && (len <= 10 || (len <= 64 && lines * len <= 1 << 21));
       // rows: as many lines as fill half a CU's LDS (two workgroups then
       // hide each other's loads), at least one; columns: a power of two of
       // them (64-byte runs at 8), fewer when the lines are long
-      if (len > kLimMax || lines / stride > 65535) {
+      if (len > kLimMax || (stride > 1 && lines / stride > 65535) || few) {
         hipLaunchKernelGGL(k_limgrad_axis, dim3(blocks_for(lines, 64)), dim3(64), 0, s, f, lines,
                            len, stride, outer, step);
       } else if (stride == 1) {

@@ -34,7 +34,11 @@ def _sweeps(f, step):
 @pytest.mark.parametrize("shape", [
     (1, 1, 1), (2, 1, 1), (1, 17, 1), (15, 16, 1), (33, 65, 1), (129, 700, 1), (700, 129, 1),
     (9300, 3, 1), (3, 9300, 1), (16384, 2, 1), (16385, 2, 1), (2, 16385, 1), (5, 6, 7),
-    (31, 40, 77), (64, 1, 130), (1, 50, 60)])
+    (31, 40, 77), (64, 1, 130), (1, 50, 60),
+    # rows: one thread a line up to 10 values, and up to 64 of 2 M values in all
+    (10, 460, 460), (11, 460, 460), (11, 500, 381), (64, 20, 30), (65, 20, 30),
+    # more lines than 65535 along axis 0, more planes than that along axis 1
+    (20, 260, 260), (70, 256, 257), (2, 3, 65536)])
 @pytest.mark.parametrize("kind", ["steps", "ramp", "special"])
 def test_limgrad_bit_for_bit(shape, kind):
     import torch
