@@ -103,6 +103,11 @@ __global__ void k_circumgrad(const double *q1, const double *q2, const double *q
 // grid its caller makes: 4.91 ms before, 0.37 now.
 constexpr int kLimSeg = 16;     // values a thread sweeps
 constexpr int kLimMax = 16384;  // longest line held in LDS (128 KiB)
+// values a workgroup holds: of rows (with one of padding each; half a CU's
+// LDS) and of columns, or one line, and the dynamic LDS that takes at most
+constexpr int kLimRows = 9216, kLimColumns = 18432;
+constexpr int kLimRowsLds = (kLimMax + 1) * (int)sizeof(double);
+constexpr int kLimColumnsLds = kLimColumns * (int)sizeof(double);
 
 // The sweeps of `lines` lines of `len` values held in LDS with stride `ls`
 // (line l at l * ll): every thread of the workgroup takes segments.
@@ -299,20 +304,22 @@ extern "C" int sm_limgrad(double *f, int nz, int nx, int ny, double elen, double
         hipLaunchKernelGGL(k_limgrad_axis, dim3(blocks_for(lines, 64)), dim3(64), 0, s, f, lines,
                            len, stride, outer, step);
       } else if (stride == 1) {
-        int per = 9216 / (len + 1);
+        int per = kLimRows / (len + 1);
         per = per < 1 ? 1 : (per > 64 ? 64 : per);
         const size_t lds = (size_t)per * (len + 1) * sizeof(double);
+        // the kernel's own bound, the same for every call: a call's own size
+        // could be another thread's too little
         SM_HIP(hipFuncSetAttribute((const void *)k_limgrad_rows,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, kLimRowsLds));
         hipLaunchKernelGGL(k_limgrad_rows, dim3((unsigned)((lines + per - 1) / per)), dim3(256),
                            lds, s, f, len, lines, per, step);
       } else {
         int per = 64;
-        while (per > 1 && (int64_t)per * len > 18432) per /= 2;
+        while (per > 1 && (int64_t)per * len > kLimColumns) per /= 2;
         while (per > 8 && (stride + per - 1) / per * (lines / stride) < 512) per /= 2;
         const size_t lds = (size_t)per * len * sizeof(double);
         SM_HIP(hipFuncSetAttribute((const void *)k_limgrad_columns,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, kLimColumnsLds));
         hipLaunchKernelGGL(k_limgrad_columns,
                            dim3((unsigned)((stride + per - 1) / per), (unsigned)(lines / stride)),
                            dim3(256), lds, s, f, len, stride, outer, per, step);
