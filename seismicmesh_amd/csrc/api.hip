@@ -129,7 +129,14 @@ __device__ inline void limit_lines(double *sh, int lines, int len, int ls, int l
         prev = v;
       }
     }
-    // then what each carries into the next, until nothing changes
+    // then what each carries into the next, until nothing changes.  The last
+    // value of a segment is read by the next one's thread while its own may
+    // lower it: a relaxed atomic, the old value or the new one (after the old
+    // one another round follows).  Reading all of them before a further
+    // barrier took 4 % longer.
+    const auto read = [&](int l, int j) {
+      return __hip_atomic_load(&at(l, j), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
     for (;;) {
       __syncthreads();
       if (threadIdx.x == 0) *changed = 0;
@@ -139,11 +146,12 @@ __device__ inline void limit_lines(double *sh, int lines, int len, int ls, int l
         int j = dir == 0 ? q * kLimSeg : (segs - q) * kLimSeg - 1;
         const int end = dir == 0 ? min(len, j + kLimSeg) : j - kLimSeg;
         const int inc = dir == 0 ? 1 : -1;
-        double prev = at(l, j - inc);
+        double prev = read(l, j - inc);
         for (int i = 0; j != end; j += inc, ++i) {
           const double lim = prev + step;
-          if (!(at(l, j) > lim)) break;
-          at(l, j) = prev = lim;
+          if (!(read(l, j) > lim)) break;
+          __hip_atomic_store(&at(l, j), lim, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          prev = lim;
           if (i == kLimSeg - 1 || j + inc == end) *changed = 1;
         }
       }
