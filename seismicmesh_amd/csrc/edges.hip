@@ -31,6 +31,7 @@ namespace {
 // kept cells is produced once, by the lower-numbered one, so every bucket is
 // free of duplicates and its offsets are the output offsets.
 struct LinkSrc {
+  static constexpr int per = 3;
   const int32_t *cells;
   const uint8_t *keep;  // optional cell mask
   const int32_t *adj;
@@ -41,6 +42,19 @@ struct LinkSrc {
     const int32_t o = adj[3 * i + (j + 2) % 3];
     if (o >= 0 && o < i && (!keep || keep[o])) return false;
     const int32_t u = cells[3 * i + j], v = cells[3 * i + (j + 1) % 3];
+    a = u < v ? u : v;
+    b = u < v ? v : u;
+    return true;
+  }
+};
+
+// Few pairs for the number of vertices: counted and scattered as they are.
+struct PairSrc {
+  static constexpr int per = 1;
+  const int32_t *pairs;
+  int64_t n;
+  __device__ inline bool get(int64_t i, int, int32_t &a, int32_t &b) const {
+    const int32_t u = pairs[2 * i], v = pairs[2 * i + 1];
     a = u < v ? u : v;
     b = u < v ? v : u;
     return true;
@@ -198,10 +212,11 @@ __global__ __launch_bounds__(kItemThreads) void k_item_scatter(int64_t n, const 
 }
 
 // cnt2 (optional): the same edges counted by their second endpoint
-__global__ void k_count(LinkSrc src, int32_t *cnt, int32_t *cnt2) {
+template <class Src>
+__global__ void k_count(Src src, int32_t *cnt, int32_t *cnt2) {
   int64_t i = (int64_t)xcd_block() * blockDim.x + threadIdx.x;
   if (i >= src.n) return;
-  for (int j = 0; j < 3; ++j) {
+  for (int j = 0; j < Src::per; ++j) {
     int32_t a, b;
     if (src.get(i, j, a, b)) {
       atomicAdd(&cnt[a], 1);
@@ -210,10 +225,11 @@ __global__ void k_count(LinkSrc src, int32_t *cnt, int32_t *cnt2) {
   }
 }
 
-__global__ void k_scatter(LinkSrc src, const int32_t *rowptr, int32_t *cur, int32_t *col) {
+template <class Src>
+__global__ void k_scatter(Src src, const int32_t *rowptr, int32_t *cur, int32_t *col) {
   int64_t i = (int64_t)xcd_block() * blockDim.x + threadIdx.x;
   if (i >= src.n) return;
-  for (int j = 0; j < 3; ++j) {
+  for (int j = 0; j < Src::per; ++j) {
     int32_t a, b;
     if (src.get(i, j, a, b)) {
       int32_t pos = rowptr[a] + atomicAdd(&cur[a], 1);
@@ -248,35 +264,75 @@ __device__ inline void sort16(int32_t (&v)[16]) {
   }
 }
 
-constexpr int kRows = 256;    // buckets of one workgroup
+constexpr int kRows = 256;    // buckets of one workgroup (and its threads)
+constexpr int kFewRows = 32;  // the same where buckets are few and long
 constexpr int kStage = 4096;  // ids staged in LDS for them
+// kFewRows buckets a workgroup up to this many buckets of 8 ids and more (1024
+// workgroups, what the chip holds at once)
+constexpr int64_t kDenseRows = 32768;
+// lists of pairs up to this long are counted as they are
+constexpr int64_t kPlainPairs = 16384;
 
-// Sorts kRows consecutive buckets and leaves each one's distinct ids,
-// ascending, at its start.  The buckets are one contiguous piece of col,
-// moved through LDS in whole lines (in global memory if it is longer than
-// kStage); a thread sorts its own bucket if short, its wave the ones of up
-// to kWaveSort ids one after the other; longer ones are listed (one atomic
-// per wave that has any) for the workgroup pass.  Listing the middle ones
-// too and sorting them in a pass of their own took 95 + 139 us on 512 k
-// lattice vertices; now 17 us.
+// Sorts one id per lane (INT32_MAX past the bucket's end wl) with a bitonic
+// network, partners exchanged by lane shuffles, and writes the distinct ids
+// to b; returns their number.
+__device__ inline int32_t sort_wave(int32_t *b, int32_t wl) {
+  const int lane = threadIdx.x % 64;
+  int32_t v = lane < wl ? b[lane] : INT32_MAX;
+#pragma unroll
+  for (int size = 2; size <= 64; size <<= 1) {
+#pragma unroll
+    for (int stride = size >> 1; stride > 0; stride >>= 1) {
+      const int32_t o = __shfl_xor(v, stride);
+      const bool up = (lane & size) == 0;
+      const bool low = (lane & stride) == 0;
+      // the lower lane of a pair keeps the smaller value in an ascending
+      // block, the larger in a descending one
+      v = (low == up) ? (v < o ? v : o) : (v < o ? o : v);
+    }
+  }
+  const int32_t prev = __shfl_up(v, 1);
+  const bool first = lane < wl && (lane == 0 || v != prev);
+  const uint64_t m = __ballot(first);
+  if (first) b[(int32_t)__popcll(m & ((1ull << lane) - 1))] = v;
+  return (int32_t)__popcll(m);
+}
+
+// Sorts R consecutive buckets and leaves each one's distinct ids, ascending,
+// at its start.  The buckets are one contiguous piece of col, moved through
+// LDS in whole lines (in global memory if it is longer than kStage or, with
+// STAGE false, for buckets of about one id, where the threads' own reads are
+// whole lines: 3 M of them 29 us through LDS, 25 without); a thread sorts its own bucket if short, a wave
+// the ones of up to kWaveSort ids one after the other; longer ones are listed
+// (one atomic per wave that has any) for the workgroup pass.  Listing the
+// middle ones too and sorting them in a pass of their own took 95 + 139 us on
+// 512 k lattice vertices; now 17 us.  R = kFewRows spreads the middle ones
+// over all waves of a workgroup: 1.7 k buckets of 20 to 60 ids, 64 of them to
+// a wave 57 us, 8 to a wave 12.
+template <int R, bool STAGE>
 __global__ __launch_bounds__(kRows) void k_row_sort(int64_t nrows, const int32_t *rowptr,
                                                     int32_t *col, int32_t *ucnt,
                                                     int32_t *long_rows, int32_t *nlong) {
-  __shared__ int32_t sh[kStage];
+  __shared__ int32_t sh[STAGE ? kStage : 1];
+  __shared__ int32_t piece[R < kRows ? R + 1 : 1];
   const int tid = threadIdx.x, lane = tid % 64;
-  const int64_t r0 = (int64_t)xcd_block() * kRows, r = r0 + tid;
+  const int64_t r0 = (int64_t)xcd_block() * R, r = r0 + tid;
   if (r == 0) ucnt[nrows] = 0;  // the scan's last input (its total slot)
   if (r0 >= nrows) return;
-  const int64_t r1 = r0 + kRows < nrows ? r0 + kRows : nrows;
-  const int32_t c0 = rowptr[r0], n = rowptr[r1] - c0;
-  const bool staged = n <= kStage;
+  const int64_t r1 = r0 + R < nrows ? r0 + R : nrows;
+  const int32_t c0 = STAGE ? rowptr[r0] : 0, n = STAGE ? rowptr[r1] - c0 : 0;
+  const bool staged = STAGE && n <= kStage;
+  if (R < kRows) {
+    if (tid <= R) piece[tid] = rowptr[r < nrows ? r : nrows] - c0;
+    __syncthreads();
+  }
   int32_t *buf = col + c0;
   if (staged) {
     for (int32_t k = tid; k < n; k += kRows) sh[k] = buf[k];
     __syncthreads();
     buf = sh;
   }
-  const bool row = r < nrows;
+  const bool row = tid < R && r < nrows;
   const int32_t s = row ? rowptr[r] - c0 : 0, len = row ? rowptr[r + 1] - c0 - s : 0;
   const uint64_t lm = __ballot(len > kWaveSort);
   if (lm) {
@@ -300,29 +356,20 @@ __global__ __launch_bounds__(kRows) void k_row_sort(int64_t nrows, const int32_t
       if (k < len && (k == 0 || v[k] != v[k - 1])) buf[s + u++] = v[k];
     ucnt[r] = u;
   }
-  // kRegSort < len <= kWaveSort: lane k holds id k (INT32_MAX past the end);
-  // a bitonic network over the 64 lanes, partners exchanged by lane shuffles
-  for (uint64_t mid = __ballot(len > kRegSort && len <= kWaveSort); mid; mid &= mid - 1) {
-    const int w = __builtin_ctzll(mid);
-    const int32_t ws = __shfl(s, w), wl = __shfl(len, w);
-    int32_t v = lane < wl ? buf[ws + lane] : INT32_MAX;
-#pragma unroll
-    for (int size = 2; size <= 64; size <<= 1) {
-#pragma unroll
-      for (int stride = size >> 1; stride > 0; stride >>= 1) {
-        const int32_t o = __shfl_xor(v, stride);
-        const bool up = (lane & size) == 0;
-        const bool low = (lane & stride) == 0;
-        // the lower lane of a pair keeps the smaller value in an ascending
-        // block, the larger in a descending one
-        v = (low == up) ? (v < o ? v : o) : (v < o ? o : v);
-      }
+  if (R < kRows) {
+    for (int w = tid / 64; w < R; w += kRows / 64) {
+      const int32_t ws = piece[w], wl = piece[w + 1] - ws;
+      if (wl <= kRegSort || wl > kWaveSort) continue;
+      const int32_t u = sort_wave(buf + ws, wl);
+      if (lane == 0) ucnt[r0 + w] = u;
     }
-    const int32_t prev = __shfl_up(v, 1);
-    const bool first = lane < wl && (lane == 0 || v != prev);
-    const uint64_t m = __ballot(first);
-    if (first) buf[ws + (int32_t)__popcll(m & ((1ull << lane) - 1))] = v;
-    if (lane == w) ucnt[r] = (int32_t)__popcll(m);
+  } else {
+    for (uint64_t mid = __ballot(len > kRegSort && len <= kWaveSort); mid; mid &= mid - 1) {
+      const int w = __builtin_ctzll(mid);
+      const int32_t ws = __shfl(s, w), wl = __shfl(len, w);
+      const int32_t u = sort_wave(buf + ws, wl);
+      if (lane == w) ucnt[r] = u;
+    }
   }
   if (!staged) return;
   __syncthreads();
@@ -524,14 +571,33 @@ int unique_edges_run(const int32_t *pairs, const int32_t *cells, const uint8_t *
   int32_t *total = count32 ? count32 : ctr + 3;
   const LinkSrc link{cells, keep, adj, n};
   const ItemSrc item{cells ? cells : pairs, keep, n};
+  // Pairs of which there is no more than one to a vertex share little that a
+  // block could drop or count together, and small lists do not pay for the
+  // tables.  (The 3 M edges of a path: 163 us through the tables, 122 as they
+  // are; in a random order 393 and 356; 1000 random pairs 58 and 50.  With
+  // 1.5 pairs to a vertex, sorted, 93 and 114; in a random order 205 and 192.)
+  const bool plain = !cells && (n <= nvert || n <= kPlainPairs);
+  const PairSrc pair{pairs, n};
   const auto items = [&](bool count) {
     int2 *list = reinterpret_cast<int2 *>(stage);
+    if (plain && count) {
+      hipLaunchKernelGGL(k_count<PairSrc>, dim3(blocks_for(n, B)), dim3(B), 0, s, pair, rowptr,
+                         (int32_t *)nullptr);
+      SM_LAUNCH_CHECK();
+      return (int)SM_OK;
+    }
+    if (plain) {
+      hipLaunchKernelGGL(k_scatter<PairSrc>, dim3(blocks_for(n, B)), dim3(B), 0, s, pair,
+                         (const int32_t *)rowptr, cur, col);
+      SM_LAUNCH_CHECK();
+      return (int)SM_OK;
+    }
     if (!cells) return item_pass<2>(item, count, rowptr, cur, list, col, s);
     if (dim == 2) return item_pass<3>(item, count, rowptr, cur, list, col, s);
     return item_pass<4>(item, count, rowptr, cur, list, col, s);
   };
   if (n > 0 && adj) {
-    hipLaunchKernelGGL(k_count, dim3(blocks_for(n, B)), dim3(B), 0, s, link, rowptr, sl.ptr);
+    hipLaunchKernelGGL(k_count<LinkSrc>, dim3(blocks_for(n, B)), dim3(B), 0, s, link, rowptr, sl.ptr);
     SM_LAUNCH_CHECK();
   } else if (n > 0 && (rc = items(true))) {
     return rc;
@@ -544,14 +610,23 @@ int unique_edges_run(const int32_t *pairs, const int32_t *cells, const uint8_t *
     rc = scan_exclusive(rowptr, rowptr, nvert + 1, adj ? total : ctr + 1, sws, s);
   if (rc) return rc;
   if (n > 0 && adj) {
-    hipLaunchKernelGGL(k_scatter, dim3(blocks_for(n, B)), dim3(B), 0, s, link, rowptr, cur, col);
+    hipLaunchKernelGGL(k_scatter<LinkSrc>, dim3(blocks_for(n, B)), dim3(B), 0, s, link,
+                       (const int32_t *)rowptr, cur, col);
     SM_LAUNCH_CHECK();
   } else if (n > 0 && (rc = items(false))) {
     return rc;
   }
   if (nvert > 0) {
-    hipLaunchKernelGGL(k_row_sort, dim3(blocks_for(nvert, kRows)), dim3(kRows), 0, s, nvert,
-                       rowptr, col, eptr, longr, ctr + 2);
+    if (!adj && nvert <= kDenseRows && npairs >= 8 * nvert)
+      hipLaunchKernelGGL((k_row_sort<kFewRows, true>), dim3(blocks_for(nvert, kFewRows)),
+                         dim3(kRows), 0, s, nvert, (const int32_t *)rowptr, col, eptr, longr,
+                         ctr + 2);
+    else if (plain && n <= nvert)
+      hipLaunchKernelGGL((k_row_sort<kRows, false>), dim3(blocks_for(nvert, kRows)), dim3(kRows), 0,
+                         s, nvert, (const int32_t *)rowptr, col, eptr, longr, ctr + 2);
+    else
+      hipLaunchKernelGGL((k_row_sort<kRows, true>), dim3(blocks_for(nvert, kRows)), dim3(kRows), 0, s,
+                         nvert, (const int32_t *)rowptr, col, eptr, longr, ctr + 2);
     SM_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_long_sorts, dim3(kLongBlocks + 1), dim3(256), 0, s, longr, ctr + 2,
                        rowptr, col, eptr, stage);

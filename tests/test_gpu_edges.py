@@ -73,3 +73,30 @@ def test_unique_edges_bucket_lengths(nv, length):
     items = rng.permutation(np.array(items))
     n = int(items.max()) + 1
     np.testing.assert_array_equal(_device(items, n), _oracle(items))
+
+
+@pytest.mark.parametrize("n,nv", [(16384, 9000), (16385, 16385), (16385, 16384), (20000, 20001)])
+@pytest.mark.parametrize("kind", ["random", "path", "equal"])
+def test_unique_edges_few_pairs(n, nv, kind):
+    # up to 16384 pairs, or one to a vertex, are counted without the tables
+    rng = np.random.default_rng(n + nv)
+    if kind == "random":
+        items = rng.integers(0, nv, (n, 2))
+    elif kind == "path":
+        i = rng.permutation(n) % (nv - 1)
+        items = np.stack([i + 1, i], 1)
+    else:
+        items = np.tile([[nv - 1, 3]], (n, 1))
+    np.testing.assert_array_equal(_device(items, nv), _oracle(items))
+
+
+@pytest.mark.parametrize("nv", [31, 32, 33, 65, 1000, 32768, 32769])
+def test_unique_edges_few_long_buckets(nv):
+    # 8 pairs to a vertex and more: up to 32768 buckets are sorted 32 to a
+    # workgroup; lengths around the per-thread, wave and workgroup sorts
+    rng = np.random.default_rng(nv)
+    first = np.repeat(np.arange(nv), rng.choice([0, 1, 16, 17, 20, 64, 65, 90], nv))
+    first = np.concatenate([first, np.full(max(0, 8 * nv + 16385 - len(first)), nv - 1)])
+    items = np.stack([first, rng.integers(0, nv, len(first))], 1)
+    items = rng.permutation(items)
+    np.testing.assert_array_equal(_device(items, nv), _oracle(items))
