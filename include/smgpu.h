@@ -365,11 +365,13 @@ int64_t sm_mesher_get_triangulation(sm_mesher *m, int32_t *tri, int32_t *adj, in
  * its points in few cells of the search grid, 7 too many or too tangled large stars, 8
  * no memory for its scratch. */
 int sm_mesher_stats(sm_mesher *m, int64_t *stats, int nstats);
-/* 3D handles: what the device build leaves to the host (small or degenerate
- * point sets) is tetrahedralised on nthreads host threads inserting the points of nslabs slabs along `axis` into one shared
- * tetrahedralisation (sm_host_delaunay3d_slabs: the serial build's cells, as
- * the device's are); its cells are copied to the device and filtered there, piece by piece, on
- * the handle's stream while the host still hands out the next pieces.
+/* 3D handles: what the device build leaves to the host (small, degenerate or
+ * strongly clustered point sets; sm_mesher_stats [15]) is tetrahedralised on
+ * nthreads host threads inserting the points of nslabs slabs along `axis` into
+ * one shared tetrahedralisation (sm_host_delaunay3d_slabs: the serial build's
+ * cells, as the device's are); its cells are copied to the device, piece by
+ * piece, on the handle's stream while the host still hands out the next
+ * pieces, and filtered there.
  * Replaces the per-rank slabs of mesh_generator.py:808-852, :867-877 and
  * decomp/blocker.py:4-111 (axis as the reference's `axis` option). */
 int sm_mesher_set_slabs(sm_mesher *m, int axis, int nslabs, int nthreads);

@@ -17,8 +17,9 @@
 // ALUs without packed instructions).  Measured on MI355X, 8192 samples, 3
 // hidden layers, eikonal term: 9.02 ms before (128 x 128 tiles on the
 // vector ALUs, 128-wide tiles also for the one-row products, separate
-// elementwise passes), 0.90 ms now, and the gradient's error against 64 bits
-// 1.5e-6 (8e-6 before).
+// elementwise passes), 0.90 ms now; the gradient's error against 64 bits, over
+// three draws of weights and samples, 5.3e-6 to 6.3e-6 before, 1.0e-6 to
+// 1.5e-6 now.
 #include <algorithm>
 
 #include "common.h"

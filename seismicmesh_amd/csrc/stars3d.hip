@@ -9,13 +9,13 @@
 //
 // One wave finds one star.  The star of v is kept as its link, a closed
 // triangulated surface around v: each lane holds one triangle (a, b, c) of
-// it (K of them in the kernel for large stars), i.e. the tetrahedron
-// (v, a, b, c), or the hull facet (v, a, b) when c is the symbolic vertex at
-// infinity.  A new point q is tested against all triangles at once: with v
-// as the origin the lifted in-sphere determinant is linear in (q, |q|^2), so
-// a triangle carries its four cofactors and their permanents, and a test is
-// eight multiply-adds against a forward error bound.  The triangles in
-// conflict are replaced by the cone from q over the rim of their hole.
+// it, i.e. the tetrahedron (v, a, b, c), or the hull facet (v, a, b) when c
+// is the symbolic vertex at infinity.  A new point q is tested against all
+// triangles at once: with v as the origin the lifted in-sphere determinant is
+// linear in (q, |q|^2), so a triangle carries its four cofactors and their
+// permanents, and a test is eight multiply-adds against a forward error
+// bound.  The triangles in conflict are replaced by the cone from q over the
+// rim of their hole.
 //   near (k_stars<false, false>): the points of the grid cells around v,
 //     sorted by distance, until every circumsphere lies in the part of the
 //     grid already seen: 85 % of the vertices of the 76-primitive solid end
@@ -28,8 +28,8 @@
 //     negative.  All open triangles share one traversal.
 // Points already refused never come back: the Voronoi cell of v only
 // shrinks.  Stars with a test inside its error bound are found again with
-// exact integer predicates (k_stars<true, true>); a degenerate lattice, with
-// many of them, goes to the host.  Vertices of more than 64 link triangles
+// exact integer predicates (k_stars<true, true>); with too many of them (a
+// lattice: most_exact_stars) the build goes to the host.  Vertices of more than 64 link triangles
 // ("hubs", 0.1 % of the vertices) get no star: their cells are found in
 // their neighbours' stars, and cells of four hubs from the triangulation of
 // the hubs alone, checked by one tree search each.  Every star emits the
@@ -39,9 +39,10 @@
 // Bound: instruction issue -- FP64 vector arithmetic, and in the tree the
 // chain of dependent node reads -- with 3 to 4 waves a SIMD to hide it.
 // Measured on MI355X, whole build (16 host threads in brackets): 523 k
-// points of the 76-primitive solid 46 ms (120-150), of which near 7.8, far
-// 33; 138 k points of a graded box model 9.6 ms (45); 3 k points of a ball
-// 0.5 ms (6.4, one thread).
+// points of the 76-primitive solid just off their lattice 27 ms (120-150), of
+// which near 7.7, far 17.5, and at the twentieth iteration, whose points lie
+// in the boundary, 46, of which near 7.8, far 33; 138 k points of a graded box
+// model 9.6 ms (45); 3 k points of a ball 0.5 ms (6.4, one thread).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -93,7 +94,6 @@ struct StarGrid {
   double lo[3], hi[3], s, inv, slack;
   int32_t g[3];
   int32_t nlev;
-  int32_t fail;
   int32_t dim[kMaxLevels][3];
   int64_t moff[kMaxLevels];
 };
@@ -422,7 +422,6 @@ struct StarLds {
 struct FarLds {
   uint32_t stack[kStack];  // tree nodes: level (3 bits), then i, j, k (9 bits each)
 };
-struct NoFarLds {};
 
 struct Tri {
   int32_t a, b, c;  // table indices; a = kDead: unused; c = kInfV: hull facet

@@ -368,11 +368,12 @@ class Mesher:
         return {name: int(s[i]) for i, name in enumerate(self.STATS)}
 
     def set_slabs(self, nslabs, axis=1, threads=None):
-        """3D: build each iteration's tetrahedralisation on `threads` host
-        threads (default: one per slab, at most the CPU count) inserting the
-        points of `nslabs` equal-width slabs along coordinate `axis` (the
-        reference's `axis` option) into one shared tetrahedralisation: the
-        cells are those of the serial build."""
+        """3D: make the tetrahedralisations that the device leaves to the
+        host (stats()["device_left"] says why) on `threads` host threads
+        (default: one per slab, at most the CPU count) inserting the points of
+        `nslabs` equal-width slabs along coordinate `axis` (the reference's
+        `axis` option) into one shared tetrahedralisation: the cells are those
+        of the serial build."""
         import os
         if threads is None:
             threads = max(1, min(int(nslabs), os.cpu_count() or 1))
