@@ -270,7 +270,8 @@ constexpr int kStage = 4096;  // ids staged in LDS for them
 // kFewRows buckets a workgroup up to this many buckets of 8 ids and more (1024
 // workgroups, what the chip holds at once)
 constexpr int64_t kDenseRows = 32768;
-// lists of pairs up to this long are counted as they are
+// lists of pairs up to this long, and fewer than 8 to a vertex, are counted as
+// they are
 constexpr int64_t kPlainPairs = 16384;
 
 // Sorts one id per lane (INT32_MAX past the bucket's end wl) with a bitonic
@@ -301,14 +302,14 @@ __device__ inline int32_t sort_wave(int32_t *b, int32_t wl) {
 // Sorts R consecutive buckets and leaves each one's distinct ids, ascending,
 // at its start.  The buckets are one contiguous piece of col, moved through
 // LDS in whole lines (in global memory if it is longer than kStage or, with
-// STAGE false, for buckets of about one id, where the threads' own reads are
-// whole lines: 3 M of them 29 us through LDS, 25 without); a thread sorts its own bucket if short, a wave
-// the ones of up to kWaveSort ids one after the other; longer ones are listed
-// (one atomic per wave that has any) for the workgroup pass.  Listing the
-// middle ones too and sorting them in a pass of their own took 95 + 139 us on
-// 512 k lattice vertices; now 17 us.  R = kFewRows spreads the middle ones
-// over all waves of a workgroup: 1.7 k buckets of 20 to 60 ids, 64 of them to
-// a wave 57 us, 8 to a wave 12.
+// STAGE false, for short lists and buckets of about one id, where the threads'
+// own reads are whole lines: 3 M of them 29 us through LDS, 25 without); a
+// thread sorts its own bucket if short, a wave the ones of up to kWaveSort
+// ids one after the other; longer ones are listed (one atomic per wave that
+// has any) for the workgroup pass.  Listing the middle ones too and sorting
+// them in a pass of their own took 95 + 139 us on 512 k lattice vertices; now
+// 17 us.  R = kFewRows spreads the middle ones over all waves of a workgroup:
+// 1.7 k buckets of 20 to 60 ids, 64 of them to a wave 57 us, 8 to a wave 12.
 template <int R, bool STAGE>
 __global__ __launch_bounds__(kRows) void k_row_sort(int64_t nrows, const int32_t *rowptr,
                                                     int32_t *col, int32_t *ucnt,
@@ -574,9 +575,10 @@ int unique_edges_run(const int32_t *pairs, const int32_t *cells, const uint8_t *
   // Pairs of which there is no more than one to a vertex share little that a
   // block could drop or count together, and small lists do not pay for the
   // tables.  (The 3 M edges of a path: 163 us through the tables, 122 as they
-  // are; in a random order 393 and 356; 1000 random pairs 58 and 50.  With
-  // 1.5 pairs to a vertex, sorted, 93 and 114; in a random order 205 and 192.)
-  const bool plain = !cells && (n <= nvert || n <= kPlainPairs);
+  // are; in a random order 393 and 356; 16 k random pairs of 5 k vertices 50
+  // and 32-37.  With 1.5 pairs to a vertex, sorted, 93 and 114; in a random
+  // order 205 and 192.  4.3 k pairs of 216 vertices 32 and 40.)
+  const bool plain = !cells && (n <= nvert || (n <= kPlainPairs && n < 8 * nvert));
   const PairSrc pair{pairs, n};
   const auto items = [&](bool count) {
     int2 *list = reinterpret_cast<int2 *>(stage);
@@ -621,7 +623,7 @@ int unique_edges_run(const int32_t *pairs, const int32_t *cells, const uint8_t *
       hipLaunchKernelGGL((k_row_sort<kFewRows, true>), dim3(blocks_for(nvert, kFewRows)),
                          dim3(kRows), 0, s, nvert, (const int32_t *)rowptr, col, eptr, longr,
                          ctr + 2);
-    else if (plain && n <= nvert)
+    else if (plain)
       hipLaunchKernelGGL((k_row_sort<kRows, false>), dim3(blocks_for(nvert, kRows)), dim3(kRows), 0,
                          s, nvert, (const int32_t *)rowptr, col, eptr, longr, ctr + 2);
     else

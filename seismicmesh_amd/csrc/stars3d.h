@@ -50,8 +50,8 @@ constexpr int64_t kStarMinPoints = 512;
 // Synchronises the stream.  *done is false when the device leaves the build
 // to the host (too few points, points in one plane, predicates its exact
 // stage cannot settle, too many uncertain ones, very large stars or points to
-// a cell of its grid, no memory for the scratch); nothing is written then that the host build does not
-// replace.
+// a cell of its grid, no memory for the scratch); nothing is written then that
+// the host build does not replace.
 int device_delaunay3d(StarScratch *sc, const double *p, int64_t n, double spacing,
                       int host_threads, int32_t *tet, int64_t cap, int64_t *count, bool *done,
                       hipStream_t s);

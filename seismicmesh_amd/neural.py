@@ -200,8 +200,8 @@ class NeuralSDF:
         """Forward and backward pass over the samples xt ((n, dim) float64
         device tensor) with targets tt (float32, distances in the network's
         frame, i.e. d * s; truncated at +-trunc when trunc > 0, where the
-        eikonal term is dropped, as it is everywhere unless eik > 0).  Fills self.grad; returns the loss
-        partials (device)."""
+        eikonal term is dropped, as it is everywhere unless eik > 0).  Fills
+        self.grad; returns the loss partials (device)."""
         n = xt.shape[0]
         # a step that is not above zero goes with no weight but 0
         drop = eik == 0 or (not eik > 0 and eik_h > 0)

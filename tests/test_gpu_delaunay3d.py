@@ -105,8 +105,8 @@ def _points(kind):
 
 @pytest.mark.parametrize("kind", [
     "random511", "random512", "random513", "random2000", "random30000", "spacing_too_large",
-    "spacing_too_small", "clustered", "box_exact", "box_noise", "box_rows", "box_rows_even", "duplicates",
-    "hub", "long", "far_from_origin", "tiny", "lattice", "plane"])
+    "spacing_too_small", "clustered", "box_exact", "box_noise", "box_rows", "box_rows_even",
+    "duplicates", "hub", "long", "far_from_origin", "tiny", "lattice", "plane"])
 def test_cells_equal_the_host_build(kind):
     p, h = _points(kind)
     p = np.ascontiguousarray(p)

@@ -75,10 +75,12 @@ def test_unique_edges_bucket_lengths(nv, length):
     np.testing.assert_array_equal(_device(items, n), _oracle(items))
 
 
-@pytest.mark.parametrize("n,nv", [(16384, 9000), (16385, 16385), (16385, 16384), (20000, 20001)])
+@pytest.mark.parametrize("n,nv", [(16384, 9000), (16385, 16385), (16385, 16384), (20000, 20001),
+                                  (4000, 500), (4000, 501)])
 @pytest.mark.parametrize("kind", ["random", "path", "equal"])
 def test_unique_edges_few_pairs(n, nv, kind):
-    # up to 16384 pairs, or one to a vertex, are counted without the tables
+    # up to 16384 pairs, fewer than 8 to a vertex, or any number up to one to a
+    # vertex are counted without the tables
     rng = np.random.default_rng(n + nv)
     if kind == "random":
         items = rng.integers(0, nv, (n, 2))
