@@ -535,26 +535,31 @@ struct Star {
   }
 
   // v, a, b (of a hull facet) and q are exactly coplanar: they share a
-  // coordinate, or three of them, q included, share two (a row along an
-  // axis).  On the edges of a box this settles what the exact stage cannot:
+  // coordinate, or (EXACT) three of them, q included, share two, a row along
+  // an axis.  On the edges of a box this settles what the exact stage cannot:
   // rows with a coordinate 0 next to neighbours at 1e-13.  (138 k points of a
   // graded box, 8 iterations from their lattice: 403 ms without the rows, 2
   // of the last 5 builds tried on the device in vain; 327 with them, all 5
-  // made there; 375 with every build on 16 host threads.)
+  // made there; 375 with every build on 16 host threads.  Looked for in the
+  // far pass too, whose uncertain points are mostly in a side, they cost it 4
+  // %.)
   __device__ bool same_plane(int a, int b, double x, double y, double z) const {
+    if ((vx == x && sh.tx[a] == x && sh.tx[b] == x) ||
+        (vy == y && sh.ty[a] == y && sh.ty[b] == y) ||
+        (vz == z && sh.tz[a] == z && sh.tz[b] == z))
+      return true;
+    if (!EXACT) return false;
     const bool vq[3] = {vx == x, vy == y, vz == z};
     const bool aq[3] = {sh.tx[a] == x, sh.ty[a] == y, sh.tz[a] == z};
     const bool bq[3] = {sh.tx[b] == x, sh.ty[b] == y, sh.tz[b] == z};
     int va = 0, vb = 0, ab = 0;
-    bool all = false;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      all = all || (vq[k] && aq[k] && bq[k]);
       va += vq[k] && aq[k];
       vb += vq[k] && bq[k];
       ab += aq[k] && bq[k];
     }
-    return all || va > 1 || vb > 1 || ab > 1;
+    return va > 1 || vb > 1 || ab > 1;
   }
 
   // lane of the finite triangle across the edge (a, b) of a hull facet
